@@ -126,7 +126,7 @@ fgpu::Sys::~Sys() {
     dfree(b); dfree(x); dfree(r); dfree(z); dfree(p); dfree(q); dfree(Ye); dfree(invd); dfree(diag);
     dfree(g); dfree(tmp); dfree(kq); dfree(gq); dfree(fslot); dfree(fval); dfree(d_dmask);
     dfree(r32); dfree(z32); dfree(p32); dfree(q32); dfree(d32); dfree(Ye32); dfree(invd32);
-    dfree(kq32); dfree(gq32); dfree(scal); dfree(part); dfree(cinv); dfree(cc); dfree(rho);
+    dfree(kq32); dfree(gq32); dfree(scal); dfree(part); dfree(ppq); dfree(cinv); dfree(cc); dfree(rho);
     dfree(cc64); dfree(cd); dfree(cres); dfree(ccoef); dfree(hist);
 }
 
@@ -719,7 +719,7 @@ extern "C" int fgpu_sys_device_bytes(const fgpu_sys *s, size_t *bytes) {
     if (!s || !bytes) return FGPU_EINVAL;
     const fgpu_mesh *m = static_cast<const fgpu_mesh *>(s->mesh);
     const size_t nd = m->n_dofs, ns = m->n_slots, nb = m->bf_cell.size(), nc = m->n_cells;
-    *bytes = nd * (11 * 8 + 1 + 6 * 4) + ns * (8 + 4) + nb * 5 * 8 + 2 * kPartRegions * (size_t)s->nb_dof * 8 +
+    *bytes = nd * (11 * 8 + 1 + 6 * 4) + ns * (8 + 4) + nb * 5 * 8 + (2 * kPartRegions * (size_t)s->nb_dof + 2 * (size_t)m->patches.n) * 8 +
              2 * kScal * 8 + (s->kq ? nc * 8 * (8 + 8 + 4 + 4) : 0) + (size_t)s->nc * s->cld * 2 + (size_t)s->nc * 12;
     return FGPU_OK;
 }
@@ -745,6 +745,8 @@ static void ensure_layout(fgpu_sys *s) {
     HIPCHECK(hipStreamSynchronize(m->ctx->stream));
     dfree(s->Ye);
     dfree(s->Ye32);
+    dfree(s->ppq);
+    s->ppq = dalloc<double>(2 * (size_t)std::max(1, m->patches.n));
     s->Ye = dalloc<double>(m->n_slots);
     s->Ye32 = dalloc<float>(m->n_slots);
     s->patch_gen = m->patch_gen;
@@ -1832,9 +1834,8 @@ template <class T>
 static void cg_iter(hipStream_t st, const Desc *D, const Desc *DC, const BatchTabs &t, int n, const SolveKind &k,
                     int reliable) {
     launch_elem<T>(st, D, t.etab, t.ne, k.coef, false, true, S_BETA, sizeof(T) == 8 ? t.lds64 : t.lds32, t.affine32);
-    launch_gather_cg<T>(st, D, t.dtab, t.nd);
     launch_scal_alpha(st, D, n);
-    launch_update_cg<T>(st, D, t.dtab, t.nd);
+    launch_cg_step<T>(st, D, t.dtab, t.nd);
     if (sizeof(T) == 4) {
         launch_coarse(st, D, nullptr, t.ctab, t.nct, 0, t.max_nc);
     } else {
@@ -1918,6 +1919,11 @@ static SolveKind make_sets(const std::vector<fgpu_sys *> &sys, std::vector<std::
     sets.assign(4, {});
     for (auto *s : sys) {
         Desc d0 = make_desc64(s, false), d1 = make_desc64(s, true), d2 = make_desc32(s, true), dc = make_desc64(s, false);
+        // the CG sets' applies leave p.q partials, one per patch
+        const int np = static_cast<const fgpu_mesh *>(s->mesh)->patches.n;
+        d0.ppq = s->ppq;
+        d2.ppq = s->ppq + np;
+        d0.n_pq = d2.n_pq = np;
         if (!k.mixed) {
             d0.pc = d1.pc = o->precond;
             if (o->precond == FGPU_PC_CHEBYSHEV) {

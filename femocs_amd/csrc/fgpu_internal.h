@@ -91,14 +91,16 @@ struct Desc {
     const void *kq, *gq;          // T, 8 per cell (stiffness / mass coefficient) or null
     const void *ua, *ub;          // T: element input u = ua + beta*ub (ub may be null)
     void *Ye;                     // T: element outputs, dof-major (see gptr/spos)
-    void *q;                      // T: gathered A u
-    void *p;                      // T: search direction (written by the CG gather)
+    void *q;                      // T: gathered A u (plain products)
+    void *p;                      // T: search direction
     const void *z;                // T: preconditioned residual
     void *x, *r, *zw;             // T: iterate, residual, preconditioned residual (written)
     const void *invdiag;          // T: 1/diag, 0 on constrained dofs
     const double *b;              // FP64 rhs (residual mode)
     double *scal;                 // kScal doubles
     double *part;                 // kPartRegions regions of nb_dof per-block partial sums
+    double *ppq;                  // CG sets: n_pq partial sums of p.q, one per patch (Q2: one
+    int n_pq;                     // per workgroup of the apply); null: the apply leaves none
     const float *metric;          // FP32 apply of tet-split meshes: 6 per cell, then |det A| per cell, or null
     // two-level preconditioner of the FP32 CG (null: Jacobi only): coarse correction c per
     // dof block (T), nc x nc inverse of the coarse operator (row-major), nc = dof blocks
@@ -123,7 +125,7 @@ struct ETab {
 };
 constexpr int kHist = 32;         // CG coefficients recorded per system for the Lanczos estimate
 constexpr int kChebMax = 12;      // largest Chebyshev degree
-constexpr int kPartRegions = 5 + kAggPerBlock;   // per descriptor set: p.q, r.z, r.r, b.b, s.c,
+constexpr int kPartRegions = 4 + kAggPerBlock;   // per descriptor set: r.z, r.r, b.b, s.c,
                                                  // aggregate sums of r (kAggPerBlock regions)
 constexpr int kCoarseRows = 16;   // coarse rows per workgroup of the coarse product
 constexpr int kCoarseMax = 8000;  // aggregates per system (their sums are staged in LDS)
@@ -202,6 +204,7 @@ struct Sys {
     // scalars and reduction scratch: [0] FP64 CG / outer, [1] FP32 inner
     double *scal = nullptr;       // 2*kScal
     double *part = nullptr;       // 2 * kPartRegions*nb_dof
+    double *ppq = nullptr;        // 2 x one p.q partial per patch (FP64 CG, FP32 CG)
     int nb_cell = 0, nb_dof = 0;
     int ppb = kPatchPerBlock;     // patches per element workgroup (tunable)
     int patch_gen = -1;           // mesh patch generation the slot buffers are sized for

@@ -10,8 +10,7 @@ template <class T> void launch_elem_diag(hipStream_t s, const Desc *D, const ETa
 void launch_elem_rhs(hipStream_t s, const Desc *D, const ETab *tab, int nblk, const double *fq, size_t lds);
 void launch_elem_vol(hipStream_t s, const Desc *D, const ETab *tab, int nblk, size_t lds);
 void launch_charge(hipStream_t s, int n, const double *b, const double *vol, double *rho);
-template <class T> void launch_gather_cg(hipStream_t s, const Desc *D, const int2 *tab, int nblk);
-template <class T> void launch_update_cg(hipStream_t s, const Desc *D, const int2 *tab, int nblk);
+template <class T> void launch_cg_step(hipStream_t s, const Desc *D, const int2 *tab, int nblk);
 template <class T> void launch_gather_res(hipStream_t s, const Desc *D, const int2 *tab, int nblk);
 template <class T> void launch_gather_plain(hipStream_t s, const Desc *D, const int2 *tab, int nblk, bool accum);
 void launch_scal_alpha(hipStream_t s, const Desc *D, int n);

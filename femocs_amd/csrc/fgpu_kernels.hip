@@ -735,6 +735,8 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
             a.nd[r] = G(d.pnodes)[n0 + jj];
         }
     };
+    // CG sets: the sum of input times output over each patch's nodes (p.q)
+    const bool want_dot = MODE == EM_APPLY && d.ppq != nullptr;
     // one patch from its loaded tables; the first one (check) leaves the workgroup early when
     // the system is idle, tested only once that patch's lists are in flight.  Returns false to
     // leave.  (Loading the next patch's tables ahead, in workgroups of several patches, was
@@ -748,7 +750,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
         const float4 *kc = a.kc, *gc = a.gc;
         const float vdet = a.vdet;
         int *eb = a.eb, *ee = a.ee, *os = a.os, *nd = a.nd;
-        (void)p;
+        double dot = 0;
         // the node lists had to arrive before the second wave is addressed: store the cell
         // entry lists meanwhile (keeps their load in the first wave)
         if constexpr (!FX) {
@@ -941,7 +943,11 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
 #pragma unroll
             for (int r = 0; r < kRounds; ++r) {
                 const int j = tid + r * kBlock;
-                if (j < np) Ye[os[r]] = finite ? (T)((double)(long long)sacc[j] * isc) : (T)__builtin_nanf("");
+                if (j < np) {
+                    const double y = finite ? (double)(long long)sacc[j] * isc : (double)__builtin_nanf("");
+                    Ye[os[r]] = (T)y;
+                    if (want_dot) dot += (double)su[j] * y;
+                }
             }
         } else {
             __syncthreads();
@@ -954,10 +960,17 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
                     T s = 0;
                     for (int e = eb[r]; e < ee[r]; ++e) s += sout[le[e]];
                     Ye[os[r]] = s;
+                    if (want_dot) dot += (double)su[j] * (double)s;
                 }
             }
         }
-        __syncthreads();
+        if (want_dot) {
+            double v[1] = {dot};
+            block_sum<1>(v);              // its barrier also ends the patch's use of LDS
+            if (tid == 0) d.ppq[p] = v[0];
+        } else {
+            __syncthreads();
+        }
         return true;
     };
     Tables a;

@@ -226,6 +226,7 @@ struct Q2Args {
     int maskin, active_only;
     const double *qm;            // tet-split form: 6 per cell (AFF kernels only)
     const unsigned char *layout; // tet-split form: 1 for an eta-flipped cell
+    double *ppq;                 // one partial of (input . output) per workgroup (the CG's p.q), or null
 };
 
 // orders a wave's LDS writes before its lanes' later reads (no other wave takes part)
@@ -416,6 +417,7 @@ __global__ __launch_bounds__(256) void k_q2_apply(Q2Args a) {
     }
     q2_wave_sync();
     // 5: back along z (thread (i, j)), one store per node into its slot
+    double dot = 0;
     if (live) {
         const int i = ta, j = tb;
         double s2[3], s2z[3];
@@ -430,7 +432,17 @@ __global__ __launch_bounds__(256) void k_q2_apply(Q2Args a) {
 #pragma unroll
             for (int q = 0; q < 3; ++q) y += kQB[q][k] * s2[q] + kQD[q][k] * s2z[q];
             a.Ye[slot[k]] = y;
+            dot += u[k] * y;
         }
+    }
+    if (a.ppq) {
+        // u . K u over the workgroup's cells, in a fixed order
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) dot += __shfl_xor(dot, o, 64);
+        __shared__ double sdot[4];
+        if (lane == 0) sdot[wv] = dot;
+        __syncthreads();
+        if (tid == 0) a.ppq[blk] = ((sdot[0] + sdot[1]) + sdot[2]) + sdot[3];
     }
 }
 
@@ -521,6 +533,7 @@ struct fgpu_q2 {
     double *b = nullptr, *x = nullptr, *r = nullptr, *z = nullptr, *p = nullptr, *q = nullptr, *Ye = nullptr;
     double *invd = nullptr, *diag = nullptr, *g = nullptr, *tmp = nullptr, *cd = nullptr, *cres = nullptr;
     double *ccoef = nullptr, *hist = nullptr, *scal = nullptr, *part = nullptr, *dflag = nullptr;
+    double *ppq = nullptr;                // p.q partials, one per workgroup of the apply
     float *invd32 = nullptr;
     unsigned char *d_dmask = nullptr;
     std::vector<unsigned char> dmask;
@@ -536,7 +549,7 @@ struct fgpu_q2 {
     int2 *d_dtab = nullptr;
     ~fgpu_q2() {
         for (double **v : {&b, &x, &r, &z, &p, &q, &Ye, &invd, &diag, &g, &tmp, &cd, &cres, &ccoef, &hist, &scal, &part,
-                           &dflag, &fslot})
+                           &dflag, &fslot, &ppq})
             q2free(*v);
         q2free(invd32);
         q2free(d_qm);
@@ -653,6 +666,9 @@ void q2_upload_tables() {
     if (dev < 64) done[dev] = true;
 }
 
+// cell blocks of the apply, a multiple of 8
+int q2_grid(int nc) { return (nc + 8 * kQ2Cells - 1) / (8 * kQ2Cells) * 8; }
+
 Desc q2_desc(fgpu_q2 *s) {
     Desc d{};
     d.n_dofs = s->n_dofs;
@@ -672,6 +688,8 @@ Desc q2_desc(fgpu_q2 *s) {
     d.b = s->b;
     d.scal = s->scal;
     d.part = s->part;
+    d.ppq = s->ppq;
+    d.n_pq = q2_grid(s->n_cells);
     d.pc = FGPU_PC_JACOBI;
     d.cd = s->cd;
     d.cres = s->cres;
@@ -715,12 +733,13 @@ void q2_ensure_metric(fgpu_q2 *s) {
     s->metric_gen = m->coord_gen;
 }
 
-void q2_apply(fgpu_q2 *s, const double *ua, const double *ub, bool maskin, bool active_only) {
+// ppq: per-workgroup partial sums of the input times the output, or null
+void q2_apply(fgpu_q2 *s, const double *ua, const double *ub, bool maskin, bool active_only, double *ppq = nullptr) {
     q2_ensure_metric(s);
     const bool aff = s->affine && s->mesh->affine_allowed;
     Q2Args a{s->n_cells, s->d_c27, s->d_spos, reinterpret_cast<const double4 *>(s->mesh->d_X64), ua, ub, s->scal,
-             s->d_dmask, s->Ye, maskin ? 1 : 0, active_only ? 1 : 0, s->d_qm, s->mesh->d_layout};
-    const int grid = (s->n_cells + 8 * kQ2Cells - 1) / (8 * kQ2Cells) * 8;   // cell blocks, a multiple of 8
+             s->d_dmask, s->Ye, maskin ? 1 : 0, active_only ? 1 : 0, s->d_qm, s->mesh->d_layout, ppq};
+    const int grid = q2_grid(s->n_cells);
     if (grid <= 0) return;
     if (aff) hipLaunchKernelGGL(k_q2_apply<true>, dim3(grid), dim3(256), 0, s->ctx->stream, a);
     else hipLaunchKernelGGL(k_q2_apply<false>, dim3(grid), dim3(256), 0, s->ctx->stream, a);
@@ -828,6 +847,7 @@ extern "C" int fgpu_q2_create(fgpu_mesh *m, fgpu_q2 **out) {
         s->hist = q2alloc<double>(2 * kHist);
         s->scal = q2alloc<double>(kScal);
         s->part = q2alloc<double>(kPartRegions * (size_t)s->nb_dof);
+        s->ppq = q2alloc<double>(std::max(q2_grid(nc), 1));
         s->dflag = q2alloc<double>(1);
         s->d_dmask = q2alloc<unsigned char>(n);
         s->d_desc = q2alloc<Desc>(1);
@@ -1102,10 +1122,9 @@ void q2_cg(fgpu_q2 *s, const fgpu_solve_opts *o, int pc, int deg, bool hist, int
         Q2CHECK(hipStreamSynchronize(st));
         if (done != 0.0) break;
         for (int it = 0; it < k; ++it) {
-            q2_apply(s, s->z, s->p, false, true);
-            launch_gather_cg<double>(st, D, s->d_dtab, s->nb_dof);
+            q2_apply(s, s->z, s->p, false, true, s->ppq);
             launch_scal_alpha(st, D, 1);
-            launch_update_cg<double>(st, D, s->d_dtab, s->nb_dof);
+            launch_cg_step<double>(st, D, s->d_dtab, s->nb_dof);
             if (pc == FGPU_PC_CHEBYSHEV) cheb();
             launch_scal_beta(st, D, 1, 0);
         }
