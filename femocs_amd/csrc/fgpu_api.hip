@@ -1002,6 +1002,7 @@ struct BatchTabs {
     const int2 *dtab = nullptr, *ctab = nullptr;
     int ne = 0, nd = 0, nct = 0;   // nct: coarse-product workgroups (systems with a coarse level)
     int max_nc = 0;                // largest coarse size of the batch (LDS of the coarse product)
+    bool fold = false;             // few enough patches in all for folded iterations
     bool affine32 = true;          // every system's FP32 descriptor uses the tet-split form
     size_t lds64 = 0, lds32 = 0;  // dynamic LDS of the element kernel, largest patch of the batch
 };
@@ -1076,6 +1077,7 @@ static BatchTabs upload_batch(fgpu_ctx *c, const std::vector<std::vector<Desc>> 
     t.nd = (int)dt.size();
     t.nct = (int)ct.size();
     t.max_nc = max_nc_b;
+    int64_t patches = 0;
     for (auto *x : sys) {
         const fgpu_mesh *m = static_cast<const fgpu_mesh *>(x->mesh);
         t.lds64 = std::max(t.lds64, patch_lds(m->patches.node_cap, m->patches.cells, sizeof(double)));
@@ -1083,7 +1085,9 @@ static BatchTabs upload_batch(fgpu_ctx *c, const std::vector<std::vector<Desc>> 
         // descriptor, which every caller builds before uploading it
         t.lds32 = std::max(t.lds32, patch_lds(m->patches.node_cap, m->patches.cells, sizeof(float), x->desc32_affine));
         t.affine32 = t.affine32 && x->desc32_affine;
+        patches += m->patches.n;
     }
+    t.fold = patches <= kFoldPatches;
     return t;
 }
 
@@ -1829,20 +1833,21 @@ static void cheb_steps(hipStream_t st, const Desc *D, const Desc *DC, const Batc
     }
 }
 
-// one CG iteration of every system of the set
+// one CG iteration of every system of the set; last: the state must be complete after it (the
+// scalar kernel that ends a folded iteration may be left out otherwise)
 template <class T>
 static void cg_iter(hipStream_t st, const Desc *D, const Desc *DC, const BatchTabs &t, int n, const SolveKind &k,
-                    int reliable) {
-    launch_elem<T>(st, D, t.etab, t.ne, k.coef, false, true, S_BETA, sizeof(T) == 8 ? t.lds64 : t.lds32, t.affine32);
-    launch_scal_alpha(st, D, n);
-    launch_cg_step<T>(st, D, t.dtab, t.nd);
+                    int reliable, bool last) {
+    launch_elem<T>(st, D, t.etab, t.ne, k.coef, false, true, S_BETA, sizeof(T) == 8 ? t.lds64 : t.lds32, t.affine32, t.fold);
+    if (!t.fold) launch_scal_alpha(st, D, n);
+    launch_cg_step<T>(st, D, t.dtab, t.nd, t.fold);
     if (sizeof(T) == 4) {
         launch_coarse(st, D, nullptr, t.ctab, t.nct, 0, t.max_nc);
     } else {
         if (k.coarse64) launch_coarse64(st, D, t.ctab, t.nct, t.max_nc);
         if (k.cheb_deg > 1) cheb_steps(st, D, DC, t, k.coef, k.cheb_deg);
     }
-    launch_scal_beta(st, D, n, reliable);
+    if (!t.fold || last) launch_scal_beta(st, D, n, reliable, t.fold);
 }
 
 // FP64 residual of the lifted system (R64: residual descriptors, u = x with the constrained
@@ -1880,10 +1885,11 @@ struct ChunkArgs {
 static void chunk(hipStream_t st, const ChunkArgs &a) {
     for (int j = 0; j < a.k; ++j) {
         if (!a.kind.mixed) {
-            cg_iter<double>(st, a.D64, a.DC, *a.t, a.n, a.kind, 0);
+            cg_iter<double>(st, a.D64, a.DC, *a.t, a.n, a.kind, 0, j + 1 == a.k);
         } else {
-            cg_iter<float>(st, a.D32, nullptr, *a.t, a.n, a.kind, 1);
-            if ((j + 1) % a.u == 0) reliable_update(st, a.D32, a.R64, *a.t, a.n, a.kind);
+            const bool update = (j + 1) % a.u == 0;
+            cg_iter<float>(st, a.D32, nullptr, *a.t, a.n, a.kind, 1, update || j + 1 == a.k);
+            if (update) reliable_update(st, a.D32, a.R64, *a.t, a.n, a.kind);
         }
     }
 }

@@ -72,6 +72,12 @@ enum Scal : int {
     S_NUPD = 16,   // reliable updates done
     S_DELTA = 17,  // reliable update when |r|^2 < S_DELTA * S_RRREF
     S_DONE = 18,   // solve finished (converged or out of iterations)
+    // folded iterations (no scalar kernels between launches, see fold_beta): what the element
+    // apply found, read by k_cg_step only
+    S_FRESH = 19,  // S_BETA and S_RZ are those of the next iteration (else: sum the partials)
+    S_GRUN = 20,   // 1: this iteration runs
+    S_GRZ = 21,    // r.z of this iteration
+    S_GBETA = 22,  // beta of this iteration
 };
 
 // Device descriptor of one system for one launch family.  Pointers are typed by the
@@ -127,6 +133,13 @@ constexpr int kHist = 32;         // CG coefficients recorded per system for the
 constexpr int kChebMax = 12;      // largest Chebyshev degree
 constexpr int kPartRegions = 4 + kAggPerBlock;   // per descriptor set: r.z, r.r, b.b, s.c,
                                                  // aggregate sums of r (kAggPerBlock regions)
+// patches of all systems of a batch up to which its CG iterations are folded (fold_beta,
+// fgpu_kernels.hip): every workgroup then sums the partials, which costs more than the two scalar
+// launches it saves once the launches are several rounds of workgroups.  Folded against not, one
+// solve: 64 patches 2.96 / 3.58 ms (FP64), 470 patches 6.2 / 7.3 (FP64) and 5.1 / 5.9 ms
+// (mixed), 1218 patches 10.1 / 10.2 and 5.8 / 6.4 ms, 1884 patches 13.2 / 13.1 and 7.3 / 7.7 ms,
+// 3656 patches 21.7 / 20.6 ms (mixed), eight tips of about 5000 in all 14.1 / 13.2 ms
+constexpr int kFoldPatches = 2048;
 constexpr int kCoarseRows = 16;   // coarse rows per workgroup of the coarse product
 constexpr int kCoarseMax = 8000;  // aggregates per system (their sums are staged in LDS)
 

@@ -256,6 +256,144 @@ template <int NV> __device__ __forceinline__ void block_sum(double (&v)[NV]) {
     }
 }
 
+// the same with the result in every thread (same bits)
+template <int NV> __device__ __forceinline__ void block_sum_all(double (&v)[NV]) {
+    __shared__ double sh[NV][kBlock / 64];
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        v[i] = wave_sum(v[i]);
+        if (lane == 0) sh[i][w] = v[i];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        double s = 0;
+#pragma unroll
+        for (int k = 0; k < kBlock / 64; ++k) s += sh[i][k];
+        v[i] = s;
+    }
+}
+
+// partial-sum regions of Desc::part (nb = nb_dof entries each)
+// (sum of r over round h of dof workgroup `block`, 256 dofs: region P_S + h, entry block)
+enum Part : int { P_RZ = 0, P_RR = 1, P_BB = 2, P_SC = 3, P_S = 4 };
+
+// sums of the partial regions of one system; valid in thread 0.  The loads of a thread are
+// independent (four accumulators), the combination order is fixed.
+__device__ __forceinline__ double thread_partials(const double *p, int n) {
+    double a0 = 0, a1 = 0, a2 = 0, a3 = 0;
+    int k = threadIdx.x;
+    for (; k + 3 * kBlock < n; k += 4 * kBlock) {
+        a0 += p[k];
+        a1 += p[k + kBlock];
+        a2 += p[k + 2 * kBlock];
+        a3 += p[k + 3 * kBlock];
+    }
+    for (; k < n; k += kBlock) a0 += p[k];
+    return (a0 + a1) + (a2 + a3);
+}
+template <int NV> __device__ __forceinline__ void sum_partials(const Desc &d, const int (&reg)[NV], double (&v)[NV]) {
+#pragma unroll
+    for (int i = 0; i < NV; ++i) v[i] = thread_partials(d.part + (size_t)reg[i] * d.nb_dof, d.nb_dof);
+    block_sum<NV>(v);
+}
+
+// r.z (with the coarse term of a two-level CG) and r.r of one system; valid in thread 0
+__device__ __forceinline__ void sum_rz_rr(const Desc &d, double (&v)[2]) {
+    if (d.cc) {
+        const int reg[3] = {P_RZ, P_RR, P_SC};
+        double w[3];
+        sum_partials<3>(d, reg, w);
+        v[0] = w[0] + w[2];
+        v[1] = w[1];
+    } else {
+        const int reg[2] = {P_RZ, P_RR};
+        sum_partials<2>(d, reg, v);
+    }
+}
+
+// whether the CG stops with |r|^2 = rr after `it` iterations (reliable: the FP32 CG of the mixed
+// solver, which also stops for a reliable update), and the state it then leaves
+__device__ __forceinline__ bool cg_stops(const double *s, double rr, double it, bool reliable) {
+    if (reliable) return rr <= s[S_THR2] || rr <= s[S_DELTA] * s[S_RRREF] || it >= s[S_MAXIT];
+    return rr <= s[S_THR2] || !(it < s[S_MAXIT]);
+}
+__device__ __forceinline__ void end_of_cg(double *s, bool reliable) {
+    s[S_ACTIVE] = 0.0;
+    if (reliable) {
+        s[S_PEND] = 1.0;
+    } else {
+        s[S_CONV] = s[S_RR] <= s[S_THR2] ? 1.0 : 0.0;
+        s[S_DONE] = 1.0;
+    }
+}
+
+// Folded iterations.  A small system spends most of an iteration between launches, so the two
+// one-workgroup scalar kernels are left out and every workgroup of the element apply and of
+// k_cg_step sums the partials itself: a few hundred doubles each, read while its own tables are
+// in flight, in the order of the scalar kernels (same bits).  No workgroup may read what another
+// of its launch writes: the apply's first workgroup leaves its findings in S_GRUN, S_GRZ, S_GBETA
+// and S_RR, which only k_cg_step reads, and k_cg_step's first workgroup updates what the apply
+// reads.
+// beta of the coming iteration in every thread; false when the CG stops instead
+__device__ __forceinline__ bool fold_beta(const Desc &d, bool lead, bool reliable, double &beta) {
+    double *s = d.scal;
+    double rz;
+    bool run = true;
+    if (s[S_FRESH] != 0.0) {
+        rz = s[S_RZ];
+        beta = s[S_BETA];
+    } else {
+        double rr;
+        if (d.cc) {
+            double v[3] = {thread_partials(d.part + (size_t)P_RZ * d.nb_dof, d.nb_dof),
+                           thread_partials(d.part + (size_t)P_RR * d.nb_dof, d.nb_dof),
+                           thread_partials(d.part + (size_t)P_SC * d.nb_dof, d.nb_dof)};
+            block_sum_all<3>(v);
+            rz = v[0] + v[2];
+            rr = v[1];
+        } else {
+            double v[2] = {thread_partials(d.part + (size_t)P_RZ * d.nb_dof, d.nb_dof),
+                           thread_partials(d.part + (size_t)P_RR * d.nb_dof, d.nb_dof)};
+            block_sum_all<2>(v);
+            rz = v[0];
+            rr = v[1];
+        }
+        beta = s[S_RZ] != 0.0 ? rz / s[S_RZ] : 0.0;
+        run = !cg_stops(s, rr, s[S_IT], reliable);
+        if (lead) {
+            s[S_RR] = rr;
+            const int j = (int)s[S_IT] - 1;
+            if (d.hist && j >= 0 && j < kHist) d.hist[2 * j + 1] = beta;
+        }
+    }
+    if (lead) {
+        s[S_GRUN] = run ? 1.0 : 0.0;
+        s[S_GRZ] = rz;
+        s[S_GBETA] = beta;
+    }
+    return run;
+}
+// alpha of this iteration in every thread, and the state of the next one
+__device__ __forceinline__ double fold_alpha(const Desc &d, bool lead) {
+    double v[1] = {thread_partials(d.ppq, d.n_pq)};
+    block_sum_all<1>(v);
+    double *s = d.scal;
+    const double rz = s[S_GRZ];
+    const double alpha = v[0] != 0.0 ? rz / v[0] : 0.0;
+    if (lead) {
+        const int j = (int)s[S_IT];
+        if (d.hist && j < kHist) d.hist[2 * j] = alpha;
+        s[S_PQ] = v[0];
+        s[S_ALPHA] = alpha;
+        s[S_RZ] = rz;
+        s[S_IT] = j + 1.0;
+        s[S_FRESH] = 0.0;
+    }
+    return alpha;
+}
+
 // the dof's element outputs sit contiguously in the slot buffer, in ascending cell order
 // Global-memory views of the descriptor's pointers: loads and stores through them are
 // global_load/global_store (scalar base + vector offset) instead of flat accesses, which also
@@ -655,7 +793,7 @@ void launch_metric(hipStream_t s, int nc, const int *cells, const unsigned char 
 // compiled in, which frees registers for more resident waves)
 template <class T, bool COEF, bool MASKIN, bool ACTIVE_ONLY, int MODE, bool AFF = false>
 __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const Desc *__restrict__ D, const ETab *__restrict__ tab, int scal_slot,
-                                                     const double *__restrict__ fq) {
+                                                     const double *__restrict__ fq, int fold) {
     constexpr int kRounds = (kPatchNodes + kBlock - 1) / kBlock;
     const ETab t = tab[blockIdx.x];
     if (t.nc == 0) return;
@@ -683,7 +821,7 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
     const auto ua = G(reinterpret_cast<const T *>(d.ua));
     const T *ub = reinterpret_cast<const T *>(d.ub);
     // converted where it is used, after the first loads are in flight
-    const double beta64 = MODE == EM_APPLY ? G(d.scal)[scal_slot] : 0.0;   // used only with ub
+    double beta64 = MODE == EM_APPLY ? G(d.scal)[scal_slot] : 0.0;   // used only with ub
     const auto Ye = GW(reinterpret_cast<T *>(d.Ye));
     const int tid = threadIdx.x;
     // A patch's first wave of loads: its tables (cell local ids, entry lists, metric and
@@ -737,13 +875,11 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
     };
     // CG sets: the sum of input times output over each patch's nodes (p.q)
     const bool want_dot = MODE == EM_APPLY && d.ppq != nullptr;
-    // one patch from its loaded tables; the first one (check) leaves the workgroup early when
-    // the system is idle, tested only once that patch's lists are in flight.  Returns false to
-    // leave.  (Loading the next patch's tables ahead, in workgroups of several patches, was
+    // one patch from its loaded tables.  (Loading the next patch's tables ahead, in workgroups of several patches, was
     // measured: the extra registers cost more resident waves than the hidden latency gained.
     // Loading only its node ids ahead keeps 8 waves resident and changed nothing: the scattered
     // node accesses cost memory requests, not latency.)
-    auto patch = [&](Tables &a, const int p, const int c0, const int nc, const int n0, const int np, const bool check) -> bool {
+    auto patch = [&](Tables &a, const int p, const int c0, const int nc, const int n0, const int np) {
         const uint4 packed = a.packed;
         const uint4 lent = a.lent;
         const float2 *mq = a.mq;
@@ -756,7 +892,6 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
         if constexpr (!FX) {
             if (tid < nc) slent[tid] = lent;
         }
-        if (ACTIVE_ONLY && check && active == 0.0) return false;   // uniform: the workgroup leaves
         const T beta = (T)beta64;
         T va[kRounds], vb[kRounds], vc[kRounds];
         unsigned char mk[kRounds];
@@ -971,17 +1106,27 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
         } else {
             __syncthreads();
         }
-        return true;
     };
     Tables a;
     load_tables(a, t.p, t.c0, t.nc, t.n0, t.np);
-    if (!patch(a, t.p, t.c0, t.nc, t.n0, t.np, true)) return;
+    // an idle system is left here, with the first patch's lists in flight (uniform)
+    if constexpr (ACTIVE_ONLY) {
+        const bool lead = t.p == 0 && tid == 0;
+        if (active == 0.0) {
+            if (fold && lead) d.scal[S_GRUN] = 0.0;
+            return;
+        }
+        if constexpr (MODE == EM_APPLY && !MASKIN) {
+            if (fold && !fold_beta(d, lead, FX, beta64)) return;
+        }
+    }
+    patch(a, t.p, t.c0, t.nc, t.n0, t.np);
     const int p_end = min(d.n_patch, t.p + d.ppb);
     for (int p = t.p + 1; p < p_end; ++p) {
         const int c0 = G(d.pcell0)[p], n0 = G(d.pnode0)[p];
         const int nc = G(d.pcell0)[p + 1] - c0, np = G(d.pnode0)[p + 1] - n0;
         load_tables(a, p, c0, nc, n0, np);
-        patch(a, p, c0, nc, n0, np, false);
+        patch(a, p, c0, nc, n0, np);
     }
 }
 
@@ -1381,17 +1526,17 @@ __global__ __launch_bounds__(kBlock) void k_grad_export(int n, const int *__rest
 // ---------------------------------------------------------------------------------------
 template <class T>
 void launch_elem(hipStream_t s, const Desc *D, const ETab *tab, int nblk, bool coef, bool maskin, bool active_only, int scal_slot,
-                 size_t lds, bool affine_all) {
+                 size_t lds, bool affine_all, bool fold) {
     if (nblk <= 0) return;
     const dim3 g(nblk), b(kBlock);
     if (sizeof(T) == 4 && affine_all && !maskin) {
-#define FG_AFF(C, A) hipLaunchKernelGGL((k_patch<T, C, false, A, EM_APPLY, true>), g, b, lds, s, D, tab, scal_slot, nullptr)
+#define FG_AFF(C, A) hipLaunchKernelGGL((k_patch<T, C, false, A, EM_APPLY, true>), g, b, lds, s, D, tab, scal_slot, nullptr, fold ? 1 : 0)
         if (coef) { if (active_only) FG_AFF(true, true); else FG_AFF(true, false); }
         else { if (active_only) FG_AFF(false, true); else FG_AFF(false, false); }
 #undef FG_AFF
         return;
     }
-#define FG_ELEM(C, M, A) hipLaunchKernelGGL((k_patch<T, C, M, A, EM_APPLY>), g, b, lds, s, D, tab, scal_slot, nullptr)
+#define FG_ELEM(C, M, A) hipLaunchKernelGGL((k_patch<T, C, M, A, EM_APPLY>), g, b, lds, s, D, tab, scal_slot, nullptr, fold ? 1 : 0)
     if (coef) {
         if (maskin) { if (active_only) FG_ELEM(true, true, true); else FG_ELEM(true, true, false); }
         else { if (active_only) FG_ELEM(true, false, true); else FG_ELEM(true, false, false); }
@@ -1401,23 +1546,23 @@ void launch_elem(hipStream_t s, const Desc *D, const ETab *tab, int nblk, bool c
     }
 #undef FG_ELEM
 }
-template void launch_elem<double>(hipStream_t, const Desc *, const ETab *, int, bool, bool, bool, int, size_t, bool);
-template void launch_elem<float>(hipStream_t, const Desc *, const ETab *, int, bool, bool, bool, int, size_t, bool);
+template void launch_elem<double>(hipStream_t, const Desc *, const ETab *, int, bool, bool, bool, int, size_t, bool, bool);
+template void launch_elem<float>(hipStream_t, const Desc *, const ETab *, int, bool, bool, bool, int, size_t, bool, bool);
 
 template <class T> void launch_elem_diag(hipStream_t s, const Desc *D, const ETab *tab, int nblk, bool coef, size_t lds) {
     if (nblk <= 0) return;
-    if (coef) hipLaunchKernelGGL((k_patch<T, true, false, false, EM_DIAG>), dim3(nblk), dim3(kBlock), lds, s, D, tab, 0, nullptr);
-    else hipLaunchKernelGGL((k_patch<T, false, false, false, EM_DIAG>), dim3(nblk), dim3(kBlock), lds, s, D, tab, 0, nullptr);
+    if (coef) hipLaunchKernelGGL((k_patch<T, true, false, false, EM_DIAG>), dim3(nblk), dim3(kBlock), lds, s, D, tab, 0, nullptr, 0);
+    else hipLaunchKernelGGL((k_patch<T, false, false, false, EM_DIAG>), dim3(nblk), dim3(kBlock), lds, s, D, tab, 0, nullptr, 0);
 }
 template void launch_elem_diag<double>(hipStream_t, const Desc *, const ETab *, int, bool, size_t);
 
 void launch_elem_rhs(hipStream_t s, const Desc *D, const ETab *tab, int nblk, const double *fq, size_t lds) {
-    if (nblk > 0) hipLaunchKernelGGL((k_patch<double, false, false, false, EM_RHS>), dim3(nblk), dim3(kBlock), lds, s, D, tab, 0, fq);
+    if (nblk > 0) hipLaunchKernelGGL((k_patch<double, false, false, false, EM_RHS>), dim3(nblk), dim3(kBlock), lds, s, D, tab, 0, fq, 0);
 }
 
 // per slot the volume of its cell (the dof volumes once gathered)
 void launch_elem_vol(hipStream_t s, const Desc *D, const ETab *tab, int nblk, size_t lds) {
-    if (nblk > 0) hipLaunchKernelGGL((k_patch<double, false, false, false, EM_VOL>), dim3(nblk), dim3(kBlock), lds, s, D, tab, 0, nullptr);
+    if (nblk > 0) hipLaunchKernelGGL((k_patch<double, false, false, false, EM_VOL>), dim3(nblk), dim3(kBlock), lds, s, D, tab, 0, nullptr, 0);
 }
 
 static inline int grid_for(int n) { return (n + kBlock - 1) / kBlock; }

@@ -1124,9 +1124,9 @@ void q2_cg(fgpu_q2 *s, const fgpu_solve_opts *o, int pc, int deg, bool hist, int
         for (int it = 0; it < k; ++it) {
             q2_apply(s, s->z, s->p, false, true, s->ppq);
             launch_scal_alpha(st, D, 1);
-            launch_cg_step<double>(st, D, s->d_dtab, s->nb_dof);
+            launch_cg_step<double>(st, D, s->d_dtab, s->nb_dof, false);
             if (pc == FGPU_PC_CHEBYSHEV) cheb();
-            launch_scal_beta(st, D, 1, 0);
+            launch_scal_beta(st, D, 1, 0, false);
         }
         Q2CHECK(hipGetLastError());
     }
