@@ -1001,7 +1001,6 @@ struct BatchTabs {
     const ETab *etab = nullptr;
     const int2 *dtab = nullptr, *ctab = nullptr;
     int ne = 0, nd = 0, nct = 0;   // nct: coarse-product workgroups (systems with a coarse level)
-    int max_nc = 0;                // largest coarse size of the batch (LDS of the coarse product)
     bool fold = false;             // few enough patches in all for folded iterations
     bool affine32 = true;          // every system's FP32 descriptor uses the tet-split form
     size_t lds64 = 0, lds32 = 0;  // dynamic LDS of the element kernel, largest patch of the batch
@@ -1017,7 +1016,6 @@ static size_t patch_lds(int node_cap, int cells, size_t tsize, bool affine = fal
 static BatchTabs upload_batch(fgpu_ctx *c, const std::vector<std::vector<Desc>> &sets, const std::vector<fgpu_sys *> &sys,
                               void **own_buf = nullptr, size_t *own_cap = nullptr) {
     std::vector<int2> et0, dt, ct;
-    int max_nc_b = 0;
     std::vector<ETab> et;
     for (size_t i = 0; i < sys.size(); ++i) {
         et0.clear();
@@ -1036,8 +1034,8 @@ static BatchTabs upload_batch(fgpu_ctx *c, const std::vector<std::vector<Desc>> 
         }
         append_table(dt, (int)i, sys[i]->nb_dof);
         if (sys[i]->coarse) {
-            for (int b = 0; b < (sys[i]->nc + kCoarseRows - 1) / kCoarseRows; ++b) ct.push_back(make_int2((int)i, b));
-            max_nc_b = std::max(max_nc_b, sys[i]->nc);
+            const int rows = coarse_rows(sys[i]->cld);
+            for (int b = 0; b < (sys[i]->nc + rows - 1) / rows; ++b) ct.push_back(make_int2((int)i, b));
         }
     }
     const size_t n = sys.size();
@@ -1076,7 +1074,6 @@ static BatchTabs upload_batch(fgpu_ctx *c, const std::vector<std::vector<Desc>> 
     t.ne = (int)et.size();
     t.nd = (int)dt.size();
     t.nct = (int)ct.size();
-    t.max_nc = max_nc_b;
     int64_t patches = 0;
     for (auto *x : sys) {
         const fgpu_mesh *m = static_cast<const fgpu_mesh *>(x->mesh);
@@ -1700,6 +1697,8 @@ static int build_coarse(fgpu_sys *s, int shift) {
     s->cc64 = dalloc<double>(nc);
     launch_to_half(st, nc, ld, dA, cscale, s->cinv);
     HIPCHECK(hipMemsetAsync(s->cc, 0, nc * sizeof(float), st));
+    // the coarse partials of another aggregate size would stay in the sums over their region
+    HIPCHECK(hipMemsetAsync(s->part, 0, 2 * kPartRegions * (size_t)s->nb_dof * sizeof(double), st));
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(st));
     dfree(dA);
@@ -1842,9 +1841,9 @@ static void cg_iter(hipStream_t st, const Desc *D, const Desc *DC, const BatchTa
     if (!t.fold) launch_scal_alpha(st, D, n);
     launch_cg_step<T>(st, D, t.dtab, t.nd, t.fold);
     if (sizeof(T) == 4) {
-        launch_coarse(st, D, nullptr, t.ctab, t.nct, 0, t.max_nc);
+        launch_coarse(st, D, nullptr, t.ctab, t.nct, 0);
     } else {
-        if (k.coarse64) launch_coarse64(st, D, t.ctab, t.nct, t.max_nc);
+        if (k.coarse64) launch_coarse64(st, D, t.ctab, t.nct);
         if (k.cheb_deg > 1) cheb_steps(st, D, DC, t, k.coef, k.cheb_deg);
     }
     if (!t.fold || last) launch_scal_beta(st, D, n, reliable, t.fold);
@@ -1858,7 +1857,7 @@ static void fp64_residual(hipStream_t st, const Desc *R64, const Desc *D32, cons
     launch_elem<double>(st, R64, t.etab, t.ne, k.coef, true, true, S_BETA, t.lds64);
     launch_gather_res<double>(st, R64, t.dtab, t.nd);
     if (!mixed) {
-        if (k.coarse64) launch_coarse64(st, R64, t.ctab, t.nct, t.max_nc);
+        if (k.coarse64) launch_coarse64(st, R64, t.ctab, t.nct);
         if (k.cheb_deg > 1) cheb_steps(st, R64, DC, t, k.coef, k.cheb_deg);
     }
     launch_scal_res(st, R64, D32, n, mixed);
@@ -1871,7 +1870,7 @@ static void reliable_update(hipStream_t st, const Desc *D32, const Desc *R64, co
     launch_mixed_acc(st, D32, R64, t.dtab, t.nd);
     fp64_residual(st, R64, D32, nullptr, t, n, k, 1);
     launch_mixed_restart(st, D32, R64, t.dtab, t.nd, 0);
-    launch_coarse(st, D32, R64, t.ctab, t.nct, 2, t.max_nc);
+    launch_coarse(st, D32, R64, t.ctab, t.nct, 2);
     launch_scal_restart(st, D32, R64, n, 0);
 }
 
@@ -1998,7 +1997,7 @@ static void start_solves(fgpu_ctx *c, const std::vector<fgpu_sys *> &sys, const 
     fp64_residual(c->stream, R64, D32, DC, t, n, k, mixed ? 1 : 0);
     if (mixed) {
         launch_mixed_restart(c->stream, D32, R64, t.dtab, t.nd, 1);
-        launch_coarse(c->stream, D32, R64, t.ctab, t.nct, 1, t.max_nc);
+        launch_coarse(c->stream, D32, R64, t.ctab, t.nct, 1);
         launch_scal_restart(c->stream, D32, R64, n, 1);
     }
     HIPCHECK(hipGetLastError());
@@ -2473,7 +2472,7 @@ static double time_launches(fgpu_ctx *c, const Desc *D, const BatchTabs &t, bool
     if (which == 2 && (precision != FGPU_MIXED || t.nct == 0)) throw std::invalid_argument("no coarse level in the batch");
     auto one = [&] {
         if (which == 2) {
-            launch_coarse(c->stream, D, nullptr, t.ctab, t.nct, 0, t.max_nc);
+            launch_coarse(c->stream, D, nullptr, t.ctab, t.nct, 0);
         } else if (which == 0) {
             if (precision == FGPU_MIXED)
                 launch_elem<float>(c->stream, D, t.etab, t.ne, coef, false, false, S_BETA, t.lds32, t.affine32);

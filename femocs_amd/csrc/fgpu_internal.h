@@ -17,7 +17,7 @@ constexpr int kBlock = 256;   // threads per workgroup (4 wave64)
 constexpr int kDofIter = 4;   // dofs per thread in the per-dof kernels
 constexpr int kDofBlock = kBlock * kDofIter;
 // coarse aggregates of the two-level preconditioner: 2^agg_shift consecutive internal dofs, a
-// multiple of kAggMin (one round of a dof workgroup: its sums of r are kept per round)
+// multiple of kAggMin (one round of a dof workgroup) and at most its dofs
 constexpr int kAggMin = kBlock;
 constexpr int kAggPerBlock = kDofIter;
 constexpr int kPatchCells = 256;  // largest patch: cells per element workgroup (one per thread)
@@ -140,8 +140,13 @@ constexpr int kPartRegions = 4 + kAggPerBlock;   // per descriptor set: r.z, r.r
 // (mixed), 1218 patches 10.1 / 10.2 and 5.8 / 6.4 ms, 1884 patches 13.2 / 13.1 and 7.3 / 7.7 ms,
 // 3656 patches 21.7 / 20.6 ms (mixed), eight tips of about 5000 in all 14.1 / 13.2 ms
 constexpr int kFoldPatches = 2048;
-constexpr int kCoarseRows = 16;   // coarse rows per workgroup of the coarse product
-constexpr int kCoarseMax = 8000;  // aggregates per system (their sums are staged in LDS)
+constexpr int kCoarseGroup = 4;   // coarse rows a wave (or several) of the coarse product forms
+// waves that share a group's rows of ld entries (a lane takes eight at a time): enough that a lane
+// reads one or two octets of a row; by the system alone, so a row's sum keeps its order in any batch
+__host__ __device__ inline int coarse_waves(int ld) { return ld <= 512 ? 1 : (ld <= 1024 ? 2 : 4); }
+// coarse rows per workgroup
+__host__ __device__ inline int coarse_rows(int ld) { return kCoarseGroup * (kBlock / 64 / coarse_waves(ld)); }
+constexpr int kCoarseMax = 8000;  // aggregates per system
 
 struct Mesh {
     fgpu_ctx *ctx = nullptr;

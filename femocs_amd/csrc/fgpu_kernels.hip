@@ -275,8 +275,8 @@ template <int NV> __device__ __forceinline__ void block_sum_all(double (&v)[NV])
     }
 }
 
-// partial-sum regions of Desc::part (nb = nb_dof entries each)
-// (sum of r over round h of dof workgroup `block`, 256 dofs: region P_S + h, entry block)
+// partial-sum regions of Desc::part (nb_dof entries each); from P_S on, the sums of r over
+// the aggregates of a two-level CG
 enum Part : int { P_RZ = 0, P_RR = 1, P_BB = 2, P_SC = 3, P_S = 4 };
 
 // sums of the partial regions of one system; valid in thread 0.  The loads of a thread are
@@ -299,18 +299,12 @@ template <int NV> __device__ __forceinline__ void sum_partials(const Desc &d, co
     block_sum<NV>(v);
 }
 
-// r.z (with the coarse term of a two-level CG) and r.r of one system; valid in thread 0
-__device__ __forceinline__ void sum_rz_rr(const Desc &d, double (&v)[2]) {
-    if (d.cc) {
-        const int reg[3] = {P_RZ, P_RR, P_SC};
-        double w[3];
-        sum_partials<3>(d, reg, w);
-        v[0] = w[0] + w[2];
-        v[1] = w[1];
-    } else {
-        const int reg[2] = {P_RZ, P_RR};
-        sum_partials<2>(d, reg, v);
-    }
+// r.z (with the coarse term of a two-level CG) and r.r of one system: each thread's share of the
+// partials, then the sums (block_sum: valid in thread 0, block_sum_all: in every thread)
+__device__ __forceinline__ void rz_rr_share(const Desc &d, double (&w)[3]) {
+    w[0] = thread_partials(d.part + (size_t)P_RZ * d.nb_dof, d.nb_dof);
+    w[1] = thread_partials(d.part + (size_t)P_RR * d.nb_dof, d.nb_dof);
+    w[2] = d.cc ? thread_partials(d.part + (size_t)P_SC * d.nb_dof, d.nb_dof) : 0.0;
 }
 
 // whether the CG stops with |r|^2 = rr after `it` iterations (reliable: the FP32 CG of the mixed
@@ -345,21 +339,11 @@ __device__ __forceinline__ bool fold_beta(const Desc &d, bool lead, bool reliabl
         rz = s[S_RZ];
         beta = s[S_BETA];
     } else {
-        double rr;
-        if (d.cc) {
-            double v[3] = {thread_partials(d.part + (size_t)P_RZ * d.nb_dof, d.nb_dof),
-                           thread_partials(d.part + (size_t)P_RR * d.nb_dof, d.nb_dof),
-                           thread_partials(d.part + (size_t)P_SC * d.nb_dof, d.nb_dof)};
-            block_sum_all<3>(v);
-            rz = v[0] + v[2];
-            rr = v[1];
-        } else {
-            double v[2] = {thread_partials(d.part + (size_t)P_RZ * d.nb_dof, d.nb_dof),
-                           thread_partials(d.part + (size_t)P_RR * d.nb_dof, d.nb_dof)};
-            block_sum_all<2>(v);
-            rz = v[0];
-            rr = v[1];
-        }
+        double w[3];
+        rz_rr_share(d, w);
+        block_sum_all<3>(w);
+        rz = w[0] + w[2];
+        const double rr = w[1];
         beta = s[S_RZ] != 0.0 ? rz / s[S_RZ] : 0.0;
         run = !cg_stops(s, rr, s[S_IT], reliable);
         if (lead) {
