@@ -998,6 +998,12 @@ static void *ensure_tab(fgpu_ctx *c, size_t bytes) {
 // [ndesc_sets x n Desc][elem table][dof table]
 struct BatchTabs {
     std::vector<const Desc *> sets;  // device pointers of each descriptor set
+    std::vector<Desc> one;           // one system alone: its descriptor of each set
+    const Desc *host(const Desc *set) const {
+        for (size_t k = 0; k < one.size(); ++k)
+            if (sets[k] == set) return &one[k];
+        return nullptr;
+    }
     const ETab *etab = nullptr;
     const int2 *dtab = nullptr, *ctab = nullptr;
     int ne = 0, nd = 0, nct = 0;   // nct: coarse-product workgroups (systems with a coarse level)
@@ -1068,6 +1074,8 @@ static BatchTabs upload_batch(fgpu_ctx *c, const std::vector<std::vector<Desc>> 
     stage_h2d(c, dev, host.data(), total);
     BatchTabs t;
     for (size_t k = 0; k < sets.size(); ++k) t.sets.push_back(reinterpret_cast<const Desc *>(dev + k * n * sizeof(Desc)));
+    if (n == 1)
+        for (auto &set : sets) t.one.push_back(set[0]);
     t.etab = reinterpret_cast<const ETab *>(dev + off_e);
     t.dtab = reinterpret_cast<const int2 *>(dev + off_d);
     t.ctab = reinterpret_cast<const int2 *>(dev + off_c);
@@ -1827,8 +1835,8 @@ struct SolveKind {
 // systems' CG or residual descriptors, DC: the same with the Chebyshev search vector as input)
 static void cheb_steps(hipStream_t st, const Desc *D, const Desc *DC, const BatchTabs &t, bool coef, int deg) {
     for (int j = 1; j < deg; ++j) {
-        launch_elem<double>(st, DC, t.etab, t.ne, coef, false, true, S_BETA, t.lds64);
-        launch_gather_cheb(st, D, t.dtab, t.nd, j);
+        launch_elem<double>(st, DC, t.etab, t.ne, coef, false, true, S_BETA, t.lds64, false, false, t.host(DC));
+        launch_gather_cheb(st, D, t.dtab, t.nd, j, t.host(D));
     }
 }
 
@@ -1837,16 +1845,18 @@ static void cheb_steps(hipStream_t st, const Desc *D, const Desc *DC, const Batc
 template <class T>
 static void cg_iter(hipStream_t st, const Desc *D, const Desc *DC, const BatchTabs &t, int n, const SolveKind &k,
                     int reliable, bool last) {
-    launch_elem<T>(st, D, t.etab, t.ne, k.coef, false, true, S_BETA, sizeof(T) == 8 ? t.lds64 : t.lds32, t.affine32, t.fold);
-    if (!t.fold) launch_scal_alpha(st, D, n);
-    launch_cg_step<T>(st, D, t.dtab, t.nd, t.fold);
+    const Desc *one = t.host(D);
+    launch_elem<T>(st, D, t.etab, t.ne, k.coef, false, true, S_BETA, sizeof(T) == 8 ? t.lds64 : t.lds32, t.affine32, t.fold,
+                   one);
+    if (!t.fold) launch_scal_alpha(st, D, n, one);
+    launch_cg_step<T>(st, D, t.dtab, t.nd, t.fold, one);
     if (sizeof(T) == 4) {
-        launch_coarse(st, D, nullptr, t.ctab, t.nct, 0);
+        launch_coarse(st, D, nullptr, t.ctab, t.nct, 0, one);
     } else {
-        if (k.coarse64) launch_coarse64(st, D, t.ctab, t.nct);
+        if (k.coarse64) launch_coarse64(st, D, t.ctab, t.nct, one);
         if (k.cheb_deg > 1) cheb_steps(st, D, DC, t, k.coef, k.cheb_deg);
     }
-    if (!t.fold || last) launch_scal_beta(st, D, n, reliable, t.fold);
+    if (!t.fold || last) launch_scal_beta(st, D, n, reliable, t.fold, one);
 }
 
 // FP64 residual of the lifted system (R64: residual descriptors, u = x with the constrained

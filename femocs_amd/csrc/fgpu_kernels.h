@@ -3,26 +3,28 @@
 #include "fgpu_internal.h"
 
 namespace fgpu {
+// one (here and below): the host copy of the descriptor of a launch for one system alone, or null
 template <class T>
 void launch_elem(hipStream_t s, const Desc *D, const ETab *tab, int nblk, bool coef, bool maskin, bool active_only,
-                 int scal_slot, size_t lds, bool affine_all = false, bool fold = false);
+                 int scal_slot, size_t lds, bool affine_all = false, bool fold = false, const Desc *one = nullptr);
 template <class T> void launch_elem_diag(hipStream_t s, const Desc *D, const ETab *tab, int nblk, bool coef, size_t lds);
 void launch_elem_rhs(hipStream_t s, const Desc *D, const ETab *tab, int nblk, const double *fq, size_t lds);
 void launch_elem_vol(hipStream_t s, const Desc *D, const ETab *tab, int nblk, size_t lds);
 void launch_charge(hipStream_t s, int n, const double *b, const double *vol, double *rho);
-template <class T> void launch_cg_step(hipStream_t s, const Desc *D, const int2 *tab, int nblk, bool fold);
+template <class T> void launch_cg_step(hipStream_t s, const Desc *D, const int2 *tab, int nblk, bool fold, const Desc *one = nullptr);
 template <class T> void launch_gather_res(hipStream_t s, const Desc *D, const int2 *tab, int nblk);
 template <class T> void launch_gather_plain(hipStream_t s, const Desc *D, const int2 *tab, int nblk, bool accum);
-void launch_scal_alpha(hipStream_t s, const Desc *D, int n);
-void launch_scal_beta(hipStream_t s, const Desc *D, int n, int reliable, bool counted);
+void launch_scal_alpha(hipStream_t s, const Desc *D, int n, const Desc *one = nullptr);
+void launch_scal_beta(hipStream_t s, const Desc *D, int n, int reliable, bool counted, const Desc *one = nullptr);
 void launch_scal_res(hipStream_t s, const Desc *D, const Desc *D32, int n, int mixed);
 void launch_scal_restart(hipStream_t s, const Desc *D32, const Desc *D64, int n, int first);
 void launch_mixed_restart(hipStream_t s, const Desc *D32, const Desc *D64, const int2 *tab, int nblk, int first);
 void launch_mixed_acc(hipStream_t s, const Desc *D32, const Desc *D64, const int2 *tab, int nblk);
 void launch_collect(hipStream_t s, const Desc *D, int n, int slot, double *out);
-void launch_coarse(hipStream_t s, const Desc *D32, const Desc *D64, const int2 *tab, int nblk, int mode);
-void launch_coarse64(hipStream_t s, const Desc *D, const int2 *tab, int nblk);
-void launch_gather_cheb(hipStream_t s, const Desc *D, const int2 *tab, int nblk, int j);
+void launch_coarse(hipStream_t s, const Desc *D32, const Desc *D64, const int2 *tab, int nblk, int mode,
+                   const Desc *one = nullptr);
+void launch_coarse64(hipStream_t s, const Desc *D, const int2 *tab, int nblk, const Desc *one = nullptr);
+void launch_gather_cheb(hipStream_t s, const Desc *D, const int2 *tab, int nblk, int j, const Desc *one = nullptr);
 void launch_coarse_indicator(hipStream_t s, int n, const unsigned char *mask, const int *color, int shift, int c,
                              double *u);
 void launch_coarse_sums(hipStream_t s, int n, const unsigned char *mask, const double *q, double *out);

@@ -331,28 +331,20 @@ __device__ __forceinline__ void end_of_cg(double *s, bool reliable) {
 // and S_RR, which only k_cg_step reads, and k_cg_step's first workgroup updates what the apply
 // reads.
 // beta of the coming iteration in every thread; false when the CG stops instead
-__device__ __forceinline__ bool fold_beta(const Desc &d, bool lead, bool reliable, double &beta) {
+// (w: rz_rr_share, read before the state is waited for)
+__device__ __forceinline__ bool fold_beta(const Desc &d, double (&w)[3], bool lead, bool reliable, double &beta) {
     double *s = d.scal;
-    double rz;
-    bool run = true;
-    if (s[S_FRESH] != 0.0) {
-        rz = s[S_RZ];
-        beta = s[S_BETA];
-    } else {
-        double w[3];
-        rz_rr_share(d, w);
-        block_sum_all<3>(w);
-        rz = w[0] + w[2];
-        const double rr = w[1];
-        beta = s[S_RZ] != 0.0 ? rz / s[S_RZ] : 0.0;
-        run = !cg_stops(s, rr, s[S_IT], reliable);
-        if (lead) {
-            s[S_RR] = rr;
+    block_sum_all<3>(w);
+    const bool fresh = s[S_FRESH] != 0.0;
+    const double rz = fresh ? s[S_RZ] : w[0] + w[2];
+    beta = fresh ? s[S_BETA] : (s[S_RZ] != 0.0 ? rz / s[S_RZ] : 0.0);
+    const bool run = fresh || !cg_stops(s, w[1], s[S_IT], reliable);
+    if (lead) {
+        if (!fresh) {
+            s[S_RR] = w[1];
             const int j = (int)s[S_IT] - 1;
             if (d.hist && j >= 0 && j < kHist) d.hist[2 * j + 1] = beta;
         }
-    }
-    if (lead) {
         s[S_GRUN] = run ? 1.0 : 0.0;
         s[S_GRZ] = rz;
         s[S_GBETA] = beta;
@@ -360,8 +352,9 @@ __device__ __forceinline__ bool fold_beta(const Desc &d, bool lead, bool reliabl
     return run;
 }
 // alpha of this iteration in every thread, and the state of the next one
-__device__ __forceinline__ double fold_alpha(const Desc &d, bool lead) {
-    double v[1] = {thread_partials(d.ppq, d.n_pq)};
+// (share: this thread's part of the p.q partials)
+__device__ __forceinline__ double fold_alpha(const Desc &d, double share, bool lead) {
+    double v[1] = {share};
     block_sum_all<1>(v);
     double *s = d.scal;
     const double rz = s[S_GRZ];
@@ -775,13 +768,10 @@ void launch_metric(hipStream_t s, int nc, const int *cells, const unsigned char 
 
 // AFF: every system of the launch has the tet-split FP32 form (the general path is not
 // compiled in, which frees registers for more resident waves)
-template <class T, bool COEF, bool MASKIN, bool ACTIVE_ONLY, int MODE, bool AFF = false>
-__global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const Desc *__restrict__ D, const ETab *__restrict__ tab, int scal_slot,
-                                                     const double *__restrict__ fq, int fold) {
+template <class T, bool COEF, bool MASKIN, bool ACTIVE_ONLY, int MODE, bool AFF>
+__device__ __forceinline__ void patch_body(const Desc &d, const ETab &t, int scal_slot, const double *__restrict__ fq, int fold) {
     constexpr int kRounds = (kPatchNodes + kBlock - 1) / kBlock;
-    const ETab t = tab[blockIdx.x];
     if (t.nc == 0) return;
-    const Desc &d = D[t.sys];
     // read now, tested once the first patch's lists are in flight (one latency fewer)
     const double active = ACTIVE_ONLY ? G(d.scal)[S_ACTIVE] : 1.0;
     using V4 = typename Vec4T<T>::type;
@@ -822,6 +812,10 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
         float4 kc[2], gc[2];
         float vdet;
         int eb[kRounds], ee[kRounds], os[kRounds], nd[kRounds];
+        // second wave of loads: the node values
+        T va[kRounds], vb[kRounds], vc[kRounds];
+        unsigned char mk[kRounds];
+        V4 xs[kRounds];
     };
     auto load_tables = [&](Tables &a, const int p, const int c0, const int nc, const int n0, const int np) {
         const int ct = tid < nc ? tid : 0;
@@ -864,7 +858,23 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
     };
     // CG sets: the sum of input times output over each patch's nodes (p.q)
     const bool want_dot = MODE == EM_APPLY && d.ppq != nullptr;
-    // one patch from its loaded tables.  (Loading the next patch's tables ahead, in workgroups of several patches, was
+    const auto ubp = G(ub ? ub : reinterpret_cast<const T *>(d.ua));   // never read through null
+    const bool cin = d.cc != nullptr && d.cc_in != 0;
+    const auto ccp = G(cin ? reinterpret_cast<const T *>(d.cc) : reinterpret_cast<const T *>(d.ua));
+    // the patch's second wave of loads: what its node ids address
+    auto load_nodes = [&](Tables &a) {
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r) {
+            if (!affine) a.xs[r] = ldg4<V4, T>(X + a.nd[r]);
+            if (MODE == EM_APPLY) {
+                a.va[r] = ua[a.nd[r]];
+                a.vb[r] = ubp[a.nd[r]];
+                a.vc[r] = ccp[cin ? a.nd[r] >> d.agg_shift : 0];
+                a.mk[r] = G(d.dmask)[a.nd[r]];
+            }
+        }
+    };
+    // one patch from its loaded tables and node values.  (Loading the next patch's tables ahead, in workgroups of several patches, was
     // measured: the extra registers cost more resident waves than the hidden latency gained.
     // Loading only its node ids ahead keeps 8 waves resident and changed nothing: the scattered
     // node accesses cost memory requests, not latency.)
@@ -874,10 +884,8 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
         const float2 *mq = a.mq;
         const float4 *kc = a.kc, *gc = a.gc;
         const float vdet = a.vdet;
-        int *eb = a.eb, *ee = a.ee, *os = a.os, *nd = a.nd;
+        int *eb = a.eb, *ee = a.ee, *os = a.os;
         double dot = 0;
-        // the node lists had to arrive before the second wave is addressed: store the cell
-        // entry lists meanwhile (keeps their load in the first wave)
         if constexpr (!FX) {
             // entry 8 cl + k: output k of cell cl, at k pcells + cl
             auto place = [&](unsigned e) { return (e & 7) * d.pcells + (e >> 3); };
@@ -885,22 +893,9 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
             if (tid < nc) slent[tid] = make_uint4(two(lent.x), two(lent.y), two(lent.z), two(lent.w));
         }
         const T beta = (T)beta64;
-        T va[kRounds], vb[kRounds], vc[kRounds];
-        unsigned char mk[kRounds];
-        V4 xs[kRounds];
-        const auto ubp = G(ub ? ub : reinterpret_cast<const T *>(d.ua));   // never read through null
-        const bool cin = d.cc != nullptr && d.cc_in != 0;
-        const auto ccp = G(cin ? reinterpret_cast<const T *>(d.cc) : reinterpret_cast<const T *>(d.ua));
-#pragma unroll
-        for (int r = 0; r < kRounds; ++r) {
-            if (!affine) xs[r] = ldg4<V4, T>(X + nd[r]);
-            if (MODE == EM_APPLY) {
-                va[r] = ua[nd[r]];
-                vb[r] = ubp[nd[r]];
-                vc[r] = ccp[cin ? nd[r] >> d.agg_shift : 0];
-                mk[r] = G(d.dmask)[nd[r]];
-            }
-        }
+        T *va = a.va, *vb = a.vb, *vc = a.vc;
+        unsigned char *mk = a.mk;
+        V4 *xs = a.xs;
 
 #pragma unroll
         for (int r = 0; r < kRounds; ++r) {
@@ -1109,16 +1104,22 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
     };
     Tables a;
     load_tables(a, t.p, t.c0, t.nc, t.n0, t.np);
+    // folded iterations: the partials, the state and the patch's lists are one wait, and the wait
+    // for the node values covers the sums
+    constexpr bool kFoldable = ACTIVE_ONLY && MODE == EM_APPLY && !MASKIN;
+    const bool lead = t.p == 0 && tid == 0;
+    double w[3] = {0, 0, 0};
+    if constexpr (kFoldable) {
+        if (fold) rz_rr_share(d, w);
+    }
     // an idle system is left here, with the first patch's lists in flight (uniform)
-    if constexpr (ACTIVE_ONLY) {
-        const bool lead = t.p == 0 && tid == 0;
-        if (active == 0.0) {
-            if (fold && lead) d.scal[S_GRUN] = 0.0;
-            return;
-        }
-        if constexpr (MODE == EM_APPLY && !MASKIN) {
-            if (fold && !fold_beta(d, lead, FX, beta64)) return;
-        }
+    if (ACTIVE_ONLY && active == 0.0) {
+        if (kFoldable && fold && lead) d.scal[S_GRUN] = 0.0;
+        return;
+    }
+    load_nodes(a);
+    if constexpr (kFoldable) {
+        if (fold && !fold_beta(d, w, lead, FX, beta64)) return;
     }
     patch(a, t.p, t.c0, t.nc, t.n0, t.np);
     const int p_end = min(d.n_patch, t.p + d.ppb);
@@ -1126,8 +1127,24 @@ __global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const 
         const int c0 = G(d.pcell0)[p], n0 = G(d.pnode0)[p];
         const int nc = G(d.pcell0)[p + 1] - c0, np = G(d.pnode0)[p + 1] - n0;
         load_tables(a, p, c0, nc, n0, np);
+        load_nodes(a);
         patch(a, p, c0, nc, n0, np);
     }
+}
+
+template <class T, bool COEF, bool MASKIN, bool ACTIVE_ONLY, int MODE, bool AFF = false>
+__global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch(const Desc *__restrict__ D, const ETab *__restrict__ tab, int scal_slot,
+                                                     const double *__restrict__ fq, int fold) {
+    const ETab t = tab[blockIdx.x];
+    patch_body<T, COEF, MASKIN, ACTIVE_ONLY, MODE, AFF>(D[t.sys], t, scal_slot, fq, fold);
+}
+// The kernels of a CG iteration of one system alone take its descriptor as an argument: it
+// arrives with the launch instead of a memory round trip after the block table's (and the
+// per-dof kernels need no table).  What a launch wrote is read by the next one from beyond the L2,
+// so each dependent access is 0.6-0.8 us of the 5-7 us that a small system's launch takes.
+template <class T, bool COEF, bool AFF>
+__global__ __launch_bounds__(kBlock, sizeof(T) == 8 ? 3 : 4) void k_patch_one(const Desc d, const ETab *__restrict__ tab, int fold) {
+    patch_body<T, COEF, false, true, EM_APPLY, AFF>(d, tab[blockIdx.x], S_BETA, nullptr, fold);
 }
 
 #include "fgpu_cg.inc"
@@ -1526,9 +1543,16 @@ __global__ __launch_bounds__(kBlock) void k_grad_export(int n, const int *__rest
 // ---------------------------------------------------------------------------------------
 template <class T>
 void launch_elem(hipStream_t s, const Desc *D, const ETab *tab, int nblk, bool coef, bool maskin, bool active_only, int scal_slot,
-                 size_t lds, bool affine_all, bool fold) {
+                 size_t lds, bool affine_all, bool fold, const Desc *one) {
     if (nblk <= 0) return;
     const dim3 g(nblk), b(kBlock);
+    // (not for the FP32 trilinear form, which spills with the descriptor in registers)
+    constexpr bool kAff = sizeof(T) == 4;
+    if (one && active_only && !maskin && scal_slot == S_BETA && (!kAff || affine_all)) {
+        if (coef) hipLaunchKernelGGL((k_patch_one<T, true, kAff>), g, b, lds, s, *one, tab, fold ? 1 : 0);
+        else hipLaunchKernelGGL((k_patch_one<T, false, kAff>), g, b, lds, s, *one, tab, fold ? 1 : 0);
+        return;
+    }
     if (sizeof(T) == 4 && affine_all && !maskin) {
 #define FG_AFF(C, A) hipLaunchKernelGGL((k_patch<T, C, false, A, EM_APPLY, true>), g, b, lds, s, D, tab, scal_slot, nullptr, fold ? 1 : 0)
         if (coef) { if (active_only) FG_AFF(true, true); else FG_AFF(true, false); }
@@ -1546,8 +1570,8 @@ void launch_elem(hipStream_t s, const Desc *D, const ETab *tab, int nblk, bool c
     }
 #undef FG_ELEM
 }
-template void launch_elem<double>(hipStream_t, const Desc *, const ETab *, int, bool, bool, bool, int, size_t, bool, bool);
-template void launch_elem<float>(hipStream_t, const Desc *, const ETab *, int, bool, bool, bool, int, size_t, bool, bool);
+template void launch_elem<double>(hipStream_t, const Desc *, const ETab *, int, bool, bool, bool, int, size_t, bool, bool, const Desc *);
+template void launch_elem<float>(hipStream_t, const Desc *, const ETab *, int, bool, bool, bool, int, size_t, bool, bool, const Desc *);
 
 template <class T> void launch_elem_diag(hipStream_t s, const Desc *D, const ETab *tab, int nblk, bool coef, size_t lds) {
     if (nblk <= 0) return;
