@@ -423,43 +423,72 @@ template <class T> __device__ __forceinline__ T coarse_term(const Desc &d, int i
 // consecutive dofs own one contiguous slot range, which the wave loads coalesced into its LDS
 // row (kWideChunk slots per pass); each lane then adds its own dof's slots from LDS in ascending
 // order.  Called by every lane of the wave; a dof past the end has the empty range at gptr[n].
-constexpr int kWideChunk = 256;
+// Latency bounds it (a wave of Q2 vertex dofs owns six times as many slots as the average one), so
+// a pass takes CHUNK slots, CHUNK / 64 loads in flight a lane, and the first 256 of the next round
+// are requested before this round's are summed.  Q2 solve of the r = 3 nm tip (720k dofs, 2.4M slots):
+// 28.2 us a Chebyshev step with 256 slots a pass and no look-ahead, 18.3 us with 1024.
 __device__ __forceinline__ void wave_lds_sync() {
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 }
-template <class T> __device__ __forceinline__ void gather_slots_wide(const Desc &d, int base, T (&q)[kDofIter]) {
-    __shared__ double wide_lds[kBlock / 64][kWideChunk];
+template <class T, int CHUNK> __device__ __forceinline__ void gather_slots_wide(const Desc &d, int base, T (&q)[kDofIter]) {
+    __shared__ double wide_lds[kBlock / 64][CHUNK];
+    constexpr int kPre = 4, kPer = CHUNK / 64;
     T *buf = reinterpret_cast<T *>(wide_lds[threadIdx.x >> 6]);
     const auto Ye = G(reinterpret_cast<const T *>(d.Ye));
     const auto gp = G(d.gptr);
     const int lane = threadIdx.x & 63, n = d.n_dofs;
+    int b[kDofIter], e[kDofIter];
 #pragma unroll
     for (int m = 0; m < kDofIter; ++m) {
         const int i = base + threadIdx.x + m * kBlock;
-        const int ic = i < n ? i : n;
-        const int b = gp[ic];
-        const int e = i < n ? gp[ic + 1] : b;
-        const int g0 = __shfl(b, 0, 64), g1 = __shfl(e, 63, 64);
+        b[m] = gp[i < n ? i : n];
+        e[m] = gp[i < n ? i + 1 : n];
+    }
+    T pre[kPre];
+    auto request = [&](int m) {
+        const int g0 = __shfl(b[m], 0, 64), g1 = __shfl(e[m], 63, 64);
+#pragma unroll
+        for (int k = 0; k < kPre; ++k) {
+            const int at = g0 + lane + 64 * k;
+            pre[k] = at < g1 ? Ye[at] : (T)0;
+        }
+    };
+    request(0);
+#pragma unroll
+    for (int m = 0; m < kDofIter; ++m) {
+        const int g0 = __shfl(b[m], 0, 64), g1 = __shfl(e[m], 63, 64);
         T s = 0;
-        for (int c0 = g0; c0 < g1; c0 += kWideChunk) {
-            const int cn = min(kWideChunk, g1 - c0);
-            for (int k = lane; k < cn; k += 64) buf[k] = Ye[c0 + k];
+        for (int c0 = g0; c0 < g1; c0 += CHUNK) {
+            const int cn = min(CHUNK, g1 - c0);
+            T v[kPer];
+#pragma unroll
+            for (int k = 0; k < kPer; ++k) {
+                if (k < kPre && c0 == g0) v[k] = pre[k];
+                else if (64 * k < cn) v[k] = lane + 64 * k < cn ? Ye[c0 + lane + 64 * k] : (T)0;
+            }
+#pragma unroll
+            for (int k = 0; k < kPer; ++k)
+                if (64 * k < cn) buf[lane + 64 * k] = v[k];
             wave_lds_sync();
-            const int lo = max(b, c0), hi = min(e, c0 + cn);
-            for (int k = lo; k < hi; ++k) s += buf[k - c0];
+            if (m + 1 < kDofIter && c0 == g0) request(m + 1);
+            const int lo = max(b[m], c0), hi = min(e[m], c0 + cn);
+            for (int k = lo; k < hi; k += 4) {          // (past the list: zeros, which change no bits)
+                T y[4];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) y[u] = buf[min(k + u, hi - 1) - c0];
+#pragma unroll
+                for (int u = 0; u < 4; ++u) s += k + u < hi ? y[u] : (T)0;
+            }
             wave_lds_sync();
         }
+        if (m + 1 < kDofIter && g0 >= g1) request(m + 1);
         q[m] = s;
     }
 }
 
 template <class T> __device__ __forceinline__ void gather_slots4(const Desc &d, int base, T (&q)[kDofIter]) {
-    if (d.wide_slots) {
-        gather_slots_wide<T>(d, base, q);
-        return;
-    }
     const auto Ye = G(reinterpret_cast<const T *>(d.Ye));
     const auto gp = G(d.gptr);
     int b[kDofIter], e[kDofIter];
@@ -484,8 +513,7 @@ template <class T> __device__ __forceinline__ void gather_slots4(const Desc &d, 
         T s = 0;
 #pragma unroll
         for (int k = 0; k < 4; ++k) s += v[m][k];
-        // long lists (Q2 vertex dofs touch about two dozen cells): four loads in flight at a
-        // time, summed in the same order
+        // long lists: four loads in flight at a time, summed in the same order
         int k = b[m] + 4;
         for (; k + 4 <= e[m]; k += 4) {
             const T y0 = Ye[k], y1 = Ye[k + 1], y2 = Ye[k + 2], y3 = Ye[k + 3];

@@ -1106,7 +1106,7 @@ void q2_cg(fgpu_q2 *s, const fgpu_solve_opts *o, int pc, int deg, bool hist, int
     auto cheb = [&] {
         for (int j = 1; j < deg; ++j) {
             q2_apply(s, s->cd, nullptr, false, true);
-            launch_gather_cheb(st, D, s->d_dtab, s->nb_dof, j);
+            launch_gather_cheb(st, D, s->d_dtab, s->nb_dof, j, &d);
         }
     };
     // residual of the lifted system and the first preconditioned residual
@@ -1123,10 +1123,10 @@ void q2_cg(fgpu_q2 *s, const fgpu_solve_opts *o, int pc, int deg, bool hist, int
         if (done != 0.0) break;
         for (int it = 0; it < k; ++it) {
             q2_apply(s, s->z, s->p, false, true, s->ppq);
-            launch_scal_alpha(st, D, 1);
-            launch_cg_step<double>(st, D, s->d_dtab, s->nb_dof, false);
+            launch_scal_alpha(st, D, 1, &d);
+            launch_cg_step<double>(st, D, s->d_dtab, s->nb_dof, false, &d);
             if (pc == FGPU_PC_CHEBYSHEV) cheb();
-            launch_scal_beta(st, D, 1, 0, false);
+            launch_scal_beta(st, D, 1, 0, false, &d);
         }
         Q2CHECK(hipGetLastError());
     }
