@@ -21,6 +21,19 @@
 
 using namespace fgpu;
 
+// The search trees as the point queries walk them: nodes in preorder (depth first, left child
+// first), two 32-byte records each.  The node after an entered one is the next record, the node
+// after a skipped one is its escape (the first node past its subtree), so the walk needs no stack,
+// and a step waits for one record instead of a box and then a child or an escape link; a subtree is
+// contiguous, so the records of a descent share cache lines.
+//   find: box of the subtree's cells (leaf: of its cell)
+//   near: box of the subtree's centroids (leaf: its centroid, three doubles in the place of the box)
+struct __align__(32) TreeNode {
+    float b[6];
+    int cell;       // the leaf's cell, -1 for an internal node
+    int escape;     // preorder position past the subtree (2 n_leaves - 1: the end)
+};
+
 struct fgpu_interp {
     fgpu_ctx *ctx = nullptr;
     int n_nodes = 0, n_tetnodes = 0, n_tets = 0, n_hexes = 0, region = 3;
@@ -31,7 +44,7 @@ struct fgpu_interp {
     double *xyz = nullptr, *det0 = nullptr, *det = nullptr, *cen = nullptr;
     int *tets = nullptr, *c10 = nullptr, *hexes = nullptr, *marker = nullptr;
     int *child = nullptr, *prim = nullptr;
-    int *esc = nullptr;                     // escape links of the tet tree
+    TreeNode *find = nullptr;        // preorder records of the tet tree (find, then near)
     float *box = nullptr, *cbox = nullptr, *leafbox = nullptr;
     int *n2c_ptr = nullptr, *n2c = nullptr, *vor_ptr = nullptr, *vor = nullptr;
     double *sol = nullptr;                  // 5 per node: vector xyz, scalar1, scalar2
@@ -58,7 +71,8 @@ struct fgpu_interp {
     LinTriHost T;
     Bvh TB;
     double *tri_tab = nullptr, *tri_cen = nullptr;
-    int *tri_child = nullptr, *tri_prim = nullptr, *tri_nodes = nullptr, *tri_esc = nullptr;
+    int *tri_child = nullptr, *tri_prim = nullptr, *tri_nodes = nullptr;
+    TreeNode *tri_find = nullptr;    // the same of the face tree
     int *tri_nbr_ptr = nullptr, *tri_nbr = nullptr;   // face neighbour lists (LinearTriangles)
     int *tri2tet = nullptr, *quad2hex = nullptr;       // the two tets of a face, hexes of a quad
     float *tri_box = nullptr, *tri_cbox = nullptr, *tri_leafbox = nullptr;
@@ -197,12 +211,11 @@ struct TriCells {
     __device__ bool searchable(int) const { return true; }
 };
 
-// Escape links of a tree (child pairs of ni internal nodes, leaves as ~leaf): for each node,
-// the node a depth-first walk visits next when it skips that node's subtree (the right sibling
-// of the nearest left child among the node and its ancestors), kBvhEnd after the last one.
-// esc[v] for internal node v, esc[ni + l] for leaf l.  The point queries walk the tree along
-// them without a stack.
-constexpr int kBvhEnd = INT_MAX;
+__device__ __forceinline__ TreeNode load_node(const TreeNode *t, int q) {
+    const float4 *p = reinterpret_cast<const float4 *>(t + q);
+    const float4 u = p[0], v = p[1];
+    return {{u.x, u.y, u.z, u.w, v.x, v.y}, __float_as_int(v.z), __float_as_int(v.w)};
+}
 __global__ __launch_bounds__(256) void kb_parents(int ni, const int *__restrict__ child, int *__restrict__ par) {
     const int v = blockIdx.x * blockDim.x + threadIdx.x;
     if (v >= ni) return;
@@ -212,64 +225,95 @@ __global__ __launch_bounds__(256) void kb_parents(int ni, const int *__restrict_
         par[c >= 0 ? c : ni + ~c] = 2 * v + k;      // position in the child array
     }
 }
-__global__ __launch_bounds__(256) void kb_escape(int ni, int nl, const int *__restrict__ child, const int *__restrict__ par,
-                                                 int *__restrict__ esc) {
+// node t: internal node t, or leaf t - ni (ni = nl - 1; leaves in left-to-right order).  A node whose
+// first leaf is f is preceded by 2 f - R nodes of subtrees to its left and its L + R ancestors
+// (reached by L left and R right turns): preorder position 2 f + L.
+__global__ __launch_bounds__(256) void kb_preorder(int nl, const int *__restrict__ child, const int *__restrict__ par,
+                                                   const float *__restrict__ box, const float *__restrict__ cbox,
+                                                   const float *__restrict__ leafbox, const int *__restrict__ prim,
+                                                   const double *__restrict__ cen, TreeNode *__restrict__ find,
+                                                   TreeNode *__restrict__ near) {
+    const int ni = nl - 1;
     const int t = blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= ni + nl) return;
-    int pe = t == 0 ? -1 : par[t];
-    int e = kBvhEnd;
-    while (pe >= 0) {
-        if ((pe & 1) == 0) {           // a left child: its right sibling is next
-            e = child[pe + 1];
-            break;
-        }
-        const int v = pe >> 1;
-        pe = v == 0 ? -1 : par[v];
+    const bool leaf = t >= ni;
+    int lefts = 0;
+    for (int v = t; v != 0;) {                       // node 0 is the root, a leaf if nl = 1
+        const int pe = par[v];
+        lefts += (pe & 1) == 0;
+        v = pe >> 1;
     }
-    esc[t] = e;
+    int f = t, l = t;
+    if (leaf) {
+        f = l = t - ni;
+    } else {
+        do f = child[2 * (size_t)f]; while (f >= 0);
+        do l = child[2 * (size_t)l + 1]; while (l >= 0);
+        f = ~f;
+        l = ~l;
+    }
+    const int pos = 2 * f + lefts;
+    TreeNode a, c;
+    a.cell = c.cell = leaf ? prim[f] : -1;
+    a.escape = c.escape = pos + 2 * (l - f) + 1;
+    const float *bx = leaf ? leafbox + 6 * (size_t)f : box + 6 * (size_t)t;
+#pragma unroll
+    for (int k = 0; k < 6; ++k) a.b[k] = bx[k];
+    if (leaf) {
+        const double x[3] = {cen[3 * (size_t)a.cell], cen[3 * (size_t)a.cell + 1], cen[3 * (size_t)a.cell + 2]};
+        __builtin_memcpy(c.b, x, sizeof(x));
+    } else {
+#pragma unroll
+        for (int k = 0; k < 6; ++k) c.b[k] = cbox[6 * (size_t)t + k];
+    }
+    find[pos] = a;
+    near[pos] = c;
 }
 
 // Per point: the lowest searchable cell containing it (x, -1 if none), the number of cells of
 // any marker containing it (y), the cell of the nearest centroid, lowest index among equal
-// distances (z, only when x < 0) and a traversal-overflow flag (w, always 0: the walk along the
-// escape links needs no stack). With `lst`, also the cells containing the point, ascending, in
+// distances (z, only when x < 0) and a traversal-overflow flag (w, always 0: the walk
+// needs no stack). With `lst`, also the cells containing the point, ascending, in
 // its row of kChainW entries (the first kChainW of them).
+// Bound by the length of the longest walks (a chain of record reads), not by bandwidth: one wave
+// per workgroup, so that few points already reach every CU.  Against separate child, escape and box
+// arrays walked by 256-thread workgroups: 301,664 points in 451,354 tets 1453 -> 678 us, 19,876 in
+// 30,515 tets 1316 -> 745 us (among 5k faces 415 -> 194 us), 1M particles 3139 -> 1920 us.
 template <class Cells>
-__global__ __launch_bounds__(256) void k_candidates(int n, const double *__restrict__ pts, int n_leaves,
-                                                    const int *__restrict__ child, const int *__restrict__ esc,
-                                                    const float *__restrict__ box,
-                                                    const float *__restrict__ cbox, const float *__restrict__ leafbox,
-                                                    const int *__restrict__ prim, Cells cells,
-                                                    const double *__restrict__ cen, int4 *__restrict__ cand,
-                                                    int *__restrict__ lst, const int *__restrict__ perm) {
+__global__ __launch_bounds__(64) void k_candidates(int n, const double *__restrict__ pts, int n_leaves,
+                                                   const TreeNode *__restrict__ find, const TreeNode *__restrict__ near,
+                                                   Cells cells, const double *__restrict__ cen, int4 *__restrict__ cand,
+                                                   int *__restrict__ lst, const int *__restrict__ perm) {
     // with `perm`, thread s takes point perm[s] (points in Morton order: a wave's points lie
     // close together and walk the tree alike); results go to the point's own index
     const int s = blockIdx.x * blockDim.x + threadIdx.x;
     if (s >= n) return;
     const int i = perm ? perm[s] : s;
     const double p[3] = {pts[3 * (size_t)i], pts[3 * (size_t)i + 1], pts[3 * (size_t)i + 2]};
-    const int ni = n_leaves - 1;
+    const int end = 2 * n_leaves - 1;
     int t0 = INT_MAX, cnt = 0;
     int *row = lst ? lst + (size_t)i * kChainW : nullptr;
     // nearest centroid: strict < over increasing indices in the reference's scan, i.e. the
     // lowest index among the minima
     double best = 1e100;
     int amin = 0;
-    auto consider = [&](int leaf) {
-        const int t = prim[leaf];
-        const double xx = p[0] - cen[3 * (size_t)t];
-        const double yy = p[1] - cen[3 * (size_t)t + 1];
-        const double zz = p[2] - cen[3 * (size_t)t + 2];
+    auto consider = [&](int t, const double *c) {
+        const double xx = p[0] - c[0];
+        const double yy = p[1] - c[1];
+        const double zz = p[2] - c[2];
         const double d2 = xx * xx + yy * yy + zz * zz;
         if (d2 < best || (d2 == best && t < amin)) {
             best = d2;
             amin = t;
         }
     };
-    auto leaf_hit = [&](int leaf) {
-        if (!in_box(leafbox + 6 * (size_t)leaf, p)) return;
-        consider(leaf);                 // the cells near the point seed the nearest-centroid search
-        const int t = prim[leaf];
+    for (int q = 0; q < end;) {
+        const TreeNode v = load_node(find, q);
+        const bool in = in_box(v.b, p);
+        q = in ? q + 1 : v.escape;      // past a leaf both are the next node
+        if (!in || v.cell < 0) continue;
+        const int t = v.cell;
+        consider(t, cen + 3 * (size_t)t);    // the cells near the point seed the nearest-centroid search
         if (cells.contains(p, t)) {
             if (row && cnt < kChainW) {
                 // insertion into the ascending row
@@ -283,34 +327,19 @@ __global__ __launch_bounds__(256) void k_candidates(int n, const double *__restr
             ++cnt;
             if (cells.searchable(t) && t < t0) t0 = t;
         }
-    };
-    if (n_leaves == 1) {
-        leaf_hit(0);
-    } else {
-        int ref = 0;                    // the root is always entered
-        while (ref != kBvhEnd) {
-            if (ref >= 0) {
-                ref = ref == 0 || in_box(box + 6 * (size_t)ref, p) ? child[2 * (size_t)ref] : esc[ref];
-            } else {
-                leaf_hit(~ref);
-                ref = esc[ni + ~ref];
-            }
-        }
     }
     if (t0 == INT_MAX) {
-        if (n_leaves == 1) {
-            consider(0);
-        } else {
-            // subtrees whose centroid box lies farther than the best distance so far are
-            // skipped; a lower bound, so no minimum (and no tie of lower index) is missed
-            int ref = 0;
-            while (ref != kBvhEnd) {
-                if (ref >= 0) {
-                    ref = box_d2(cbox + 6 * (size_t)ref, p) > best ? esc[ref] : child[2 * (size_t)ref];
-                } else {
-                    consider(~ref);
-                    ref = esc[ni + ~ref];
-                }
+        // subtrees whose centroid box lies farther than the best distance so far are
+        // skipped; a lower bound, so no minimum (and no tie of lower index) is missed
+        for (int q = 0; q < end;) {
+            const TreeNode v = load_node(near, q);
+            if (v.cell >= 0) {
+                double c[3];
+                __builtin_memcpy(c, v.b, sizeof(c));
+                consider(v.cell, c);
+                ++q;
+            } else {
+                q = box_d2(v.b, p) > best ? v.escape : q + 1;
             }
         }
     }
@@ -917,9 +946,10 @@ void ensure_chain(fgpu_interp *ip, size_t n) {
 void free_triangles(fgpu_interp *ip) {
     for (double **p : {&ip->tri_tab, &ip->tri_cen, &ip->quad_cen}) release(*p);
     for (int **p : {&ip->tri_child, &ip->tri_prim, &ip->tri_nodes, &ip->quad_nodes, &ip->tri6, &ip->quad_child,
-                    &ip->quad_prim, &ip->tri_esc, &ip->tri_nbr_ptr, &ip->tri_nbr, &ip->tri2tet, &ip->quad2hex})
+                    &ip->quad_prim, &ip->tri_nbr_ptr, &ip->tri_nbr, &ip->tri2tet, &ip->quad2hex})
         release(*p);
     for (float **p : {&ip->tri_box, &ip->tri_cbox, &ip->tri_leafbox, &ip->quad_cbox}) release(*p);
+    release(ip->tri_find);
     ip->T = LinTriHost{};
     ip->TB = Bvh{};
     ip->QB = Bvh{};
@@ -930,9 +960,10 @@ void free_interp(fgpu_interp *ip) {
     for (int **p : {&ip->tets, &ip->c10, &ip->hexes, &ip->marker, &ip->child, &ip->prim, &ip->n2c_ptr, &ip->n2c,
                     &ip->vor_ptr, &ip->vor, &ip->node_idof, &ip->tet, &ip->cells, &ip->cells2, &ip->d_region_hex,
                     &ip->sc_icell,
-                    &ip->d_hex_cell, &ip->d_nbr_ptr, &ip->d_nbr, &ip->esc})
+                    &ip->d_hex_cell, &ip->d_nbr_ptr, &ip->d_nbr})
         release(*p);
     for (float **p : {&ip->box, &ip->cbox, &ip->leafbox}) release(*p);
+    release(ip->find);
     release(ip->cand);
     release(ip->cand2);
     for (int **p : {&ip->chain_lst, &ip->chain_entry, &ip->chain_flag}) release(*p);
@@ -997,25 +1028,32 @@ const int *point_order(fgpu_interp *ip, int n, int n_leaves, const float *root_b
 
 void tet_candidates(fgpu_interp *ip, int n, int4 *cand, int *lst = nullptr) {
     const int *perm = point_order(ip, n, ip->B.n_leaves, ip->box);
-    hipLaunchKernelGGL(k_candidates<TetCells>, dim3(grid(n)), dim3(256), 0, ip->ctx->stream, n, ip->pts,
-                       ip->B.n_leaves, ip->child, ip->esc, ip->box, ip->cbox, ip->leafbox, ip->prim,
+    hipLaunchKernelGGL(k_candidates<TetCells>, dim3((n + 63) / 64), dim3(64), 0, ip->ctx->stream, n, ip->pts,
+                       ip->B.n_leaves, ip->find, ip->find + (2 * ip->B.n_leaves - 1),
                        TetCells{ip->det0, ip->det, ip->marker}, ip->cen, cand, lst, perm);
 }
 
-// the escape links of a tree of nl leaves (device child array) into a new array
-int *tree_escapes(hipStream_t s, int nl, const int *child) {
-    const int ni = std::max(nl - 1, 0);
-    int *esc = nullptr, *par = nullptr;
-    IPCHECK(hipMalloc(&esc, std::max<size_t>((size_t)ni + nl, 1) * sizeof(int)));
-    if (ni > 0) {
-        IPCHECK(hipMalloc(&par, ((size_t)ni + nl) * sizeof(int)));
-        hipLaunchKernelGGL(kb_parents, dim3(grid(ni)), dim3(256), 0, s, ni, child, par);
-        hipLaunchKernelGGL(kb_escape, dim3(grid(ni + nl)), dim3(256), 0, s, ni, nl, child, par, esc);
-        IPCHECK(hipGetLastError());
-        IPCHECK(hipStreamSynchronize(s));
-        IPCHECK(hipFree(par));
+// the preorder records of a tree of nl leaves (device arrays) in a new array: 2 nl - 1 find
+// records, then as many near records
+TreeNode *tree_records(hipStream_t s, int nl, const int *child, const float *box, const float *cbox, const float *leafbox,
+                       const int *prim, const double *cen) {
+    const int ni = std::max(nl - 1, 0), nn = std::max(2 * nl - 1, 0);
+    TreeNode *rec = nullptr;
+    int *par = nullptr;
+    IPCHECK(hipMalloc(&rec, std::max<size_t>(2 * (size_t)nn, 1) * sizeof(TreeNode)));
+    if (nl <= 0) return rec;
+    hipError_t e = hipMalloc(&par, (size_t)nn * sizeof(int));
+    if (e == hipSuccess) {
+        if (ni > 0) hipLaunchKernelGGL(kb_parents, dim3(grid(ni)), dim3(256), 0, s, ni, child, par);
+        hipLaunchKernelGGL(kb_preorder, dim3(grid(nn)), dim3(256), 0, s, nl, child, par, box, cbox, leafbox, prim, cen, rec,
+                           rec + nn);
+        e = hipGetLastError();
+        if (e == hipSuccess) e = hipStreamSynchronize(s);
+        (void)hipFree(par);
     }
-    return esc;
+    if (e != hipSuccess) (void)hipFree(rec);
+    IPCHECK(e);
+    return rec;
 }
 
 // the chained guess over the located points (ip->pts, n of them) into ip->tet, in the
@@ -1193,7 +1231,7 @@ extern "C" int fgpu_interp_create_ex(fgpu_ctx *c, int n_nodes, const double *xyz
             ip->vor = upload(vor.data(), vor.size(), s);
             IPCHECK(hipStreamSynchronize(s));   // the host vectors are read until the copies end
         }
-        ip->esc = tree_escapes(s, ip->B.n_leaves, ip->child);
+        ip->find = tree_records(s, ip->B.n_leaves, ip->child, ip->box, ip->cbox, ip->leafbox, ip->prim, ip->cen);
         // the nodal solution starts at the empty value everywhere (filled on the device)
         IPCHECK(hipMalloc(&ip->sol, 5 * (size_t)n_nodes * sizeof(double)));
         launch_set_const(s, 5 * n_nodes, empty_value, ip->sol);
@@ -1816,7 +1854,8 @@ extern "C" int fgpu_interp_set_triangles(fgpu_interp *ip, int n_tris, const int 
         ip->tri_box = upload(ip->TB.box.data(), ip->TB.box.size(), s);
         ip->tri_cbox = upload(ip->TB.cbox.data(), ip->TB.cbox.size(), s);
         ip->tri_leafbox = upload(ip->TB.leafbox.data(), ip->TB.leafbox.size(), s);
-        ip->tri_esc = tree_escapes(s, ip->TB.n_leaves, ip->tri_child);
+        ip->tri_find = tree_records(s, ip->TB.n_leaves, ip->tri_child, ip->tri_box, ip->tri_cbox, ip->tri_leafbox,
+                                    ip->tri_prim, ip->tri_cen);
         ip->tri_nbr_ptr = upload(ip->T.nbr_ptr.data(), ip->T.nbr_ptr.size(), s);
         ip->tri_nbr = upload(ip->T.nbr.data(), ip->T.nbr.size(), s);
         ip->tri2tet = upload(ip->T.tri2tet.data(), ip->T.tri2tet.size(), s);
@@ -1844,8 +1883,8 @@ static bool device_surface(fgpu_interp *ip, int n, int *cells, double *out, int 
     tet_candidates(ip, n, ip->cand);
     if (locate) {
         const int *perm = point_order(ip, n, ip->TB.n_leaves, ip->tri_box);
-        hipLaunchKernelGGL(k_candidates<TriCells>, dim3(grid(n)), dim3(256), 0, st, n, ip->pts, ip->TB.n_leaves,
-                           ip->tri_child, ip->tri_esc, ip->tri_box, ip->tri_cbox, ip->tri_leafbox, ip->tri_prim,
+        hipLaunchKernelGGL(k_candidates<TriCells>, dim3((n + 63) / 64), dim3(64), 0, st, n, ip->pts, ip->TB.n_leaves,
+                           ip->tri_find, ip->tri_find + (2 * ip->TB.n_leaves - 1),
                            TriCells{ip->tri_tab}, ip->tri_cen, ip->cand2, ip->chain_lst, perm);
         // the first guess: |-1| as a face, or |-1| / 3 from the quadrangle numbering
         run_chain(ip, n, ip->cand2, ip->tri_nbr_ptr, ip->tri_nbr, ip->T.n, rank == 3 ? 0 : 1, ip->cells2);
@@ -1923,9 +1962,8 @@ static int surface_run(fgpu_interp *ip, int n, const double *xyz, int rank, int 
             // more than kChainW - 1 faces, or a quadrangle pick with NaN weights)
             tet_candidates(ip, n, ip->cand);
             if (locate)
-                hipLaunchKernelGGL(k_candidates<TriCells>, dim3(grid(n)), dim3(256), 0, st, n, ip->pts,
-                                   ip->TB.n_leaves, ip->tri_child, ip->tri_esc, ip->tri_box, ip->tri_cbox,
-                                   ip->tri_leafbox, ip->tri_prim, TriCells{ip->tri_tab}, ip->tri_cen, ip->cand2,
+                hipLaunchKernelGGL(k_candidates<TriCells>, dim3((n + 63) / 64), dim3(64), 0, st, n, ip->pts,
+                                   ip->TB.n_leaves, ip->tri_find, ip->tri_find + (2 * ip->TB.n_leaves - 1), TriCells{ip->tri_tab}, ip->tri_cen, ip->cand2,
                                    nullptr, nullptr);
             IPCHECK(hipGetLastError());
             std::vector<int4> tc(n), fc(locate ? n : 0);

@@ -1,0 +1,47 @@
+"""Point search on trees of every small size (one leaf, two, ...) and across the sizes of a call:
+located cells equal the oracle's scan, on either build of the tables."""
+from types import SimpleNamespace
+
+import numpy as np
+import pytest
+
+from femocs_amd import interp
+from femocs_amd import mesh as M
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+
+
+def _part(small_mesh, k):
+    """The first k tets of the mesh around its middle, as a mesh of their own, split into hexes."""
+    c = small_mesh.nodes[small_mesh.tets].mean(1)
+    pick = np.argsort(np.linalg.norm(c - c.mean(0), axis=1), kind="stable")[:k]
+    used, tets = np.unique(small_mesh.tets[pick], return_inverse=True)
+    tets = tets.reshape(-1, 4)
+    nodes, kind, hexes = M.tet_to_hex(small_mesh.nodes[used], tets)
+    marker = np.where(np.arange(k) % 4 == 3, M.TYPES_BULK, M.TYPES_VACUUM).astype(np.int32)
+    hm = np.where(np.repeat(marker, 4) == M.TYPES_VACUUM, 1, -1).astype(np.int32)
+    return SimpleNamespace(nodes=nodes, node_kind=kind, tets=tets.astype(np.int32), tet_marker=marker,
+                           tet_nbr=M._face_neighbours(tets), hexes=hexes, hex_marker=hm)
+
+
+@pytest.mark.parametrize("host_build", [False, True])
+@pytest.mark.parametrize("k", [1, 2, 3, 4, 7, 64, 65, 300])
+@pytest.mark.parametrize("n", [1, 65, 2500])
+def test_located_cells(ctx, small_mesh, host_build, k, n):
+    part = _part(small_mesh, k)
+    ip = interp.Interpolator(ctx, part, interp.TYPES_VACUUM, host_build=host_build)
+    L = O.LinTet(part.nodes, part.tets, part.tet_nbr, part.tet_marker, 3)
+    rng = np.random.default_rng(100 * k + n)
+    P = part.nodes[part.tets]
+    t = rng.integers(0, k, n)
+    inside = (P[t] * rng.dirichlet(np.ones(4), n)[:, :, None]).sum(1)
+    lo, hi = part.nodes.min(0), part.nodes.max(0)
+    anywhere = rng.uniform(lo - 0.3 * (hi - lo), hi + 0.3 * (hi - lo), (n, 3))
+    pts = np.where(rng.random(n)[:, None] < 0.5, inside, anywhere)
+    pts[:: 7] = P[t[::7], 0]                       # on vertices: several cells hold the point
+    ip.set_nodal(rng.standard_normal((len(part.nodes), 5)))
+    cells, _ = ip.points(pts, 1)
+    ref, _ = O.interp_points(L, part.nodes, part.tets, O.quadtet_cells(part.tets, part.hexes, part.node_kind),
+                             part.hexes, ip.nodal(), pts, 1)
+    assert np.array_equal(cells, ref)
