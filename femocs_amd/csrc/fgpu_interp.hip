@@ -279,35 +279,55 @@ __global__ __launch_bounds__(256) void kb_preorder(int nl, const int *__restrict
 // per workgroup, so that few points already reach every CU.  Against separate child, escape and box
 // arrays walked by 256-thread workgroups: 301,664 points in 451,354 tets 1453 -> 678 us, 19,876 in
 // 30,515 tets 1316 -> 745 us (among 5k faces 415 -> 194 us), 1M particles 3139 -> 1920 us.
-template <class Cells>
+// kSplit lanes share a point: each walks its own stretch of the preorder (a stretch may begin below
+// a node that the whole walk would have skipped: boxes are nested, so nothing in there is entered),
+// all of them search the nearest centroid from the best one that any of them met.
+template <class Cells, int kSplit>
 __global__ __launch_bounds__(64) void k_candidates(int n, const double *__restrict__ pts, int n_leaves,
                                                    const TreeNode *__restrict__ find, const TreeNode *__restrict__ near,
                                                    Cells cells, const double *__restrict__ cen, int4 *__restrict__ cand,
                                                    int *__restrict__ lst, const int *__restrict__ perm) {
+    constexpr int kPoints = 64 / kSplit;
+    __shared__ int hits[kPoints];
+    __shared__ int held[kPoints][kSplit > 1 ? kChainW : 1];
+    const int g = threadIdx.x / kSplit, part = threadIdx.x % kSplit;
     // with `perm`, thread s takes point perm[s] (points in Morton order: a wave's points lie
     // close together and walk the tree alike); results go to the point's own index
-    const int s = blockIdx.x * blockDim.x + threadIdx.x;
-    if (s >= n) return;
-    const int i = perm ? perm[s] : s;
+    const int s = blockIdx.x * kPoints + g;
+    if (threadIdx.x < kPoints) hits[threadIdx.x] = 0;
+    __syncthreads();
+    const bool live = s < n;              // the lanes of a point agree; none leaves before the last barrier
+    const int i = live ? (perm ? perm[s] : s) : 0;
     const double p[3] = {pts[3 * (size_t)i], pts[3 * (size_t)i + 1], pts[3 * (size_t)i + 2]};
-    const int end = 2 * n_leaves - 1;
+    const int end = live ? 2 * n_leaves - 1 : 0;
+    const int q0 = (int)((long long)end * part / kSplit), q1 = (int)((long long)end * (part + 1) / kSplit);
     int t0 = INT_MAX, cnt = 0;
-    int *row = lst ? lst + (size_t)i * kChainW : nullptr;
+    int *row = lst && live ? lst + (size_t)i * kChainW : nullptr;
     // nearest centroid: strict < over increasing indices in the reference's scan, i.e. the
     // lowest index among the minima
     double best = 1e100;
     int amin = 0;
-    auto consider = [&](int t, const double *c) {
-        const double xx = p[0] - c[0];
-        const double yy = p[1] - c[1];
-        const double zz = p[2] - c[2];
-        const double d2 = xx * xx + yy * yy + zz * zz;
+    auto take = [&](double d2, int t) {
         if (d2 < best || (d2 == best && t < amin)) {
             best = d2;
             amin = t;
         }
     };
-    for (int q = 0; q < end;) {
+    auto consider = [&](int t, const double *c) {
+        const double xx = p[0] - c[0];
+        const double yy = p[1] - c[1];
+        const double zz = p[2] - c[2];
+        take(xx * xx + yy * yy + zz * zz, t);
+    };
+    auto merge_nearest = [&] {
+#pragma unroll
+        for (int o = kSplit / 2; o > 0; o >>= 1) {
+            const double d = __shfl_xor(best, o, 64);
+            const int t = __shfl_xor(amin, o, 64);
+            take(d, t);
+        }
+    };
+    for (int q = q0; q < q1;) {
         const TreeNode v = load_node(find, q);
         const bool in = in_box(v.b, p);
         q = in ? q + 1 : v.escape;      // past a leaf both are the next node
@@ -315,23 +335,45 @@ __global__ __launch_bounds__(64) void k_candidates(int n, const double *__restri
         const int t = v.cell;
         consider(t, cen + 3 * (size_t)t);    // the cells near the point seed the nearest-centroid search
         if (cells.contains(p, t)) {
-            if (row && cnt < kChainW) {
-                // insertion into the ascending row
-                int k = cnt;
-                while (k > 0 && row[k - 1] > t) {
-                    row[k] = row[k - 1];
-                    --k;
+            if constexpr (kSplit == 1) {
+                if (row && cnt < kChainW) {
+                    // insertion into the ascending row
+                    int k = cnt;
+                    while (k > 0 && row[k - 1] > t) {
+                        row[k] = row[k - 1];
+                        --k;
+                    }
+                    row[k] = t;
                 }
-                row[k] = t;
+                ++cnt;
+            } else {
+                const int k = atomicAdd(&hits[g], 1);
+                if (k < kChainW) held[g][k] = t;
             }
-            ++cnt;
             if (cells.searchable(t) && t < t0) t0 = t;
+        }
+    }
+    if constexpr (kSplit > 1) {
+#pragma unroll
+        for (int o = kSplit / 2; o > 0; o >>= 1) t0 = min(t0, __shfl_xor(t0, o, 64));
+        merge_nearest();
+        __syncthreads();
+        cnt = hits[g];
+        if (part == 0 && row) {
+            const int m = min(cnt, kChainW);
+            for (int k = 1; k < m; ++k) {            // ascending
+                const int t = held[g][k];
+                int j = k;
+                for (; j > 0 && held[g][j - 1] > t; --j) held[g][j] = held[g][j - 1];
+                held[g][j] = t;
+            }
+            for (int k = 0; k < m; ++k) row[k] = held[g][k];
         }
     }
     if (t0 == INT_MAX) {
         // subtrees whose centroid box lies farther than the best distance so far are
         // skipped; a lower bound, so no minimum (and no tie of lower index) is missed
-        for (int q = 0; q < end;) {
+        for (int q = q0; q < q1;) {
             const TreeNode v = load_node(near, q);
             if (v.cell >= 0) {
                 double c[3];
@@ -342,8 +384,9 @@ __global__ __launch_bounds__(64) void k_candidates(int n, const double *__restri
                 q = box_d2(v.b, p) > best ? v.escape : q + 1;
             }
         }
+        if constexpr (kSplit > 1) merge_nearest();   // the point's lanes are all here
     }
-    cand[i] = make_int4(t0 == INT_MAX ? -1 : t0, cnt, t0 == INT_MAX ? amin : 0, 0);
+    if (live && part == 0) cand[i] = make_int4(t0 == INT_MAX ? -1 : t0, cnt, t0 == INT_MAX ? amin : 0, 0);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1026,11 +1069,29 @@ const int *point_order(fgpu_interp *ip, int n, int n_leaves, const float *root_b
     return ip->sperm;
 }
 
+// Points up to which 16 and 8 lanes share one: few points leave most of the chip waiting for the
+// longest walks, many fill it and pay for the extra steps of the split.  Whole calls, 1 / 8 / 16 lanes
+// a point: 1,688 atoms 734 / 635 / 607 us, 19,876 atoms 1621 / 1285 / 1198 us (surface transfer 2469 /
+// 1803 / 1606), 63,293 atoms 1664 / 1621 / 1723 us, 60,000 particles 2045 / 1562 / 1515 us, 200,000
+// particles 3276 / 3221 / 3338 us, 301,664 atoms 4504 / 5131 / 5796 us
+constexpr int kSplit16 = 32768, kSplit8 = 131072;
+template <class Cells>
+void launch_candidates(hipStream_t s, int n, const double *pts, int n_leaves, const TreeNode *find, Cells cells,
+                       const double *cen, int4 *cand, int *lst, const int *perm) {
+    const TreeNode *near = find + std::max(2 * n_leaves - 1, 0);
+#define FG_CAND(S)                                                                                          \
+    hipLaunchKernelGGL((k_candidates<Cells, S>), dim3((n + 64 / S - 1) / (64 / S)), dim3(64), 0, s, n, pts, n_leaves, \
+                       find, near, cells, cen, cand, lst, perm)
+    if (n <= kSplit16) FG_CAND(16);
+    else if (n <= kSplit8) FG_CAND(8);
+    else FG_CAND(1);
+#undef FG_CAND
+}
+
 void tet_candidates(fgpu_interp *ip, int n, int4 *cand, int *lst = nullptr) {
     const int *perm = point_order(ip, n, ip->B.n_leaves, ip->box);
-    hipLaunchKernelGGL(k_candidates<TetCells>, dim3((n + 63) / 64), dim3(64), 0, ip->ctx->stream, n, ip->pts,
-                       ip->B.n_leaves, ip->find, ip->find + (2 * ip->B.n_leaves - 1),
-                       TetCells{ip->det0, ip->det, ip->marker}, ip->cen, cand, lst, perm);
+    launch_candidates(ip->ctx->stream, n, ip->pts, ip->B.n_leaves, ip->find, TetCells{ip->det0, ip->det, ip->marker}, ip->cen,
+                      cand, lst, perm);
 }
 
 // the preorder records of a tree of nl leaves (device arrays) in a new array: 2 nl - 1 find
@@ -1883,9 +1944,8 @@ static bool device_surface(fgpu_interp *ip, int n, int *cells, double *out, int 
     tet_candidates(ip, n, ip->cand);
     if (locate) {
         const int *perm = point_order(ip, n, ip->TB.n_leaves, ip->tri_box);
-        hipLaunchKernelGGL(k_candidates<TriCells>, dim3((n + 63) / 64), dim3(64), 0, st, n, ip->pts, ip->TB.n_leaves,
-                           ip->tri_find, ip->tri_find + (2 * ip->TB.n_leaves - 1),
-                           TriCells{ip->tri_tab}, ip->tri_cen, ip->cand2, ip->chain_lst, perm);
+        launch_candidates(st, n, ip->pts, ip->TB.n_leaves, ip->tri_find, TriCells{ip->tri_tab}, ip->tri_cen, ip->cand2,
+                          ip->chain_lst, perm);
         // the first guess: |-1| as a face, or |-1| / 3 from the quadrangle numbering
         run_chain(ip, n, ip->cand2, ip->tri_nbr_ptr, ip->tri_nbr, ip->T.n, rank == 3 ? 0 : 1, ip->cells2);
     } else {
@@ -1962,9 +2022,8 @@ static int surface_run(fgpu_interp *ip, int n, const double *xyz, int rank, int 
             // more than kChainW - 1 faces, or a quadrangle pick with NaN weights)
             tet_candidates(ip, n, ip->cand);
             if (locate)
-                hipLaunchKernelGGL(k_candidates<TriCells>, dim3((n + 63) / 64), dim3(64), 0, st, n, ip->pts,
-                                   ip->TB.n_leaves, ip->tri_find, ip->tri_find + (2 * ip->TB.n_leaves - 1), TriCells{ip->tri_tab}, ip->tri_cen, ip->cand2,
-                                   nullptr, nullptr);
+                launch_candidates(st, n, ip->pts, ip->TB.n_leaves, ip->tri_find, TriCells{ip->tri_tab}, ip->tri_cen,
+                                  ip->cand2, nullptr, nullptr);
             IPCHECK(hipGetLastError());
             std::vector<int4> tc(n), fc(locate ? n : 0);
             IPCHECK(hipMemcpyAsync(tc.data(), ip->cand, n * sizeof(int4), hipMemcpyDeviceToHost, st));

@@ -1,5 +1,7 @@
-"""Point search on trees of every small size (one leaf, two, ...) and across the sizes of a call:
-located cells equal the oracle's scan, on either build of the tables."""
+"""Point search on trees of every small size (one leaf, two, ...) and across the sizes of a call
+(16 lanes share a point up to 32768 points, 8 above, one above 131072): located cells equal the
+oracle's scan, on either build of the tables, and the same points in one call of each kind give
+the same cells."""
 from types import SimpleNamespace
 
 import numpy as np
@@ -27,7 +29,7 @@ def _part(small_mesh, k):
 
 @pytest.mark.parametrize("host_build", [False, True])
 @pytest.mark.parametrize("k", [1, 2, 3, 4, 7, 64, 65, 300])
-@pytest.mark.parametrize("n", [1, 65, 2500])
+@pytest.mark.parametrize("n", [1, 65, 2500, 32769])
 def test_located_cells(ctx, small_mesh, host_build, k, n):
     part = _part(small_mesh, k)
     ip = interp.Interpolator(ctx, part, interp.TYPES_VACUUM, host_build=host_build)
@@ -45,3 +47,15 @@ def test_located_cells(ctx, small_mesh, host_build, k, n):
     ref, _ = O.interp_points(L, part.nodes, part.tets, O.quadtet_cells(part.tets, part.hexes, part.node_kind),
                              part.hexes, ip.nodal(), pts, 1)
     assert np.array_equal(cells, ref)
+
+
+def test_lanes_per_point_find_the_same_cells(ctx, small_mesh):
+    ip = interp.Interpolator(ctx, small_mesh, interp.TYPES_VACUUM)
+    rng = np.random.default_rng(8)
+    lo, hi = small_mesh.nodes.min(0), small_mesh.nodes.max(0)
+    pts = rng.uniform(lo - 0.05 * (hi - lo), hi + 0.05 * (hi - lo), (131073, 3))
+    pts[::5] = small_mesh.nodes[rng.integers(0, len(small_mesh.nodes), len(pts[::5]))]
+    ip.set_nodal(np.zeros((len(small_mesh.nodes), 5)))
+    one = ip.points(pts, 1)[0]
+    for n in (131072, 32768, 777):
+        assert np.array_equal(ip.points(pts[:n], 1)[0], one[:n])
