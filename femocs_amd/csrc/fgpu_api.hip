@@ -190,6 +190,7 @@ static void ctx_free(fgpu_ctx *c) {
     }
     if (c->d_tab) (void)hipFree(c->d_tab);
     if (c->h_flags) (void)hipHostFree(c->h_flags);
+    if (c->d_flags) (void)hipFree(c->d_flags);
     for (int k = 0; k < fgpu_ctx::kStage; ++k) {
         if (c->stage_host[k]) (void)hipHostFree(c->stage_host[k]);
         if (c->stage_ev[k]) (void)hipEventDestroy(c->stage_ev[k]);
@@ -1813,6 +1814,19 @@ static double *flags_buffer(fgpu_ctx *c, size_t n) {
     return c->h_flags;
 }
 
+// the context's device flags, one per system
+static double *device_flags(fgpu_ctx *c, size_t n) {
+    if (n > c->dflags_cap) {
+        HIPCHECK(hipStreamSynchronize(c->stream));
+        if (c->d_flags) HIPCHECK(hipFree(c->d_flags));
+        c->d_flags = nullptr;
+        c->dflags_cap = 0;
+        HIPCHECK(hipMalloc(reinterpret_cast<void **>(&c->d_flags), 2 * n * sizeof(double)));
+        c->dflags_cap = 2 * n;
+    }
+    return c->d_flags;
+}
+
 // true while some system of the set has scalar `slot` equal to `want`
 static bool any_flag(fgpu_ctx *c, const Desc *D, int n, int slot, double want, double *dflags) {
     double *h = flags_buffer(c, n);
@@ -2038,32 +2052,39 @@ static void run_solves(fgpu_ctx *c, const std::vector<fgpu_sys *> &sys, const fg
     kind.coef = coef;
     BatchTabs t = upload_batch(c, sets, sys);
     start_solves(c, sys, o, t, kind);
-    double *dflags = nullptr;
-    HIPCHECK(hipMalloc(&dflags, std::max(1, n) * sizeof(double)));
+    double *dflags = device_flags(c, n);
     ChunkArgs a{kind, k, 8, n, t.sets[0], t.sets[1], t.sets[2], t.sets[3], &t};
     // a system waiting for its reliable update idles at most u iterations per update
     const int max_chunks = 2 * (max_it / k) + 16;
+    // use_graph: a chunk is captured while the second one, launched directly, runs on the GPU, and
+    // replayed from then on.  Captured before the first chunk, it kept the GPU waiting 170-250 us
+    // of every solve, also of those that end within a chunk.
     hipGraphExec_t exec = nullptr;
     hipGraph_t graph = nullptr;
+    struct Release {
+        hipGraphExec_t &exec;
+        hipGraph_t &graph;
+        ~Release() {
+            if (exec) (void)hipGraphExecDestroy(exec);
+            if (graph) (void)hipGraphDestroy(graph);
+        }
+    } release{exec, graph};
     bool running = any_flag(c, t.sets[1], n, S_DONE, 0.0, dflags);
     for (int ch = 0; running && ch < max_chunks; ++ch) {
-        if (o->use_graph) {
-            if (!exec) {
+        if (exec) {
+            HIPCHECK(hipGraphLaunch(exec, c->stream));
+        } else {
+            chunk(c->stream, a);
+            if (o->use_graph && ch > 0) {
                 HIPCHECK(hipStreamBeginCapture(c->stream, hipStreamCaptureModeThreadLocal));
                 chunk(c->stream, a);
                 HIPCHECK(hipStreamEndCapture(c->stream, &graph));
                 HIPCHECK(hipGraphInstantiate(&exec, graph, nullptr, nullptr, 0));
             }
-            HIPCHECK(hipGraphLaunch(exec, c->stream));
-        } else {
-            chunk(c->stream, a);
         }
         running = any_flag(c, t.sets[1], n, S_DONE, 0.0, dflags);
     }
-    if (exec) (void)hipGraphExecDestroy(exec);
-    if (graph) (void)hipGraphDestroy(graph);
     HIPCHECK(hipStreamSynchronize(c->stream));
-    HIPCHECK(hipFree(dflags));
     if (stats)
         for (int i = 0; i < n; ++i) read_stats(sys[i], kind.mixed, &stats[i]);
 }

@@ -288,6 +288,8 @@ struct fgpu_ctx {
     size_t tab_bytes = 0;
     double *h_flags = nullptr;    // pinned, per system
     size_t flags_cap = 0;
+    double *d_flags = nullptr;    // the same on the device
+    size_t dflags_cap = 0;
     int refs = 0;                 // live meshes and systems
     bool closing = false;         // destroy requested while children were alive
     bool affine_table = false;    // reference sub-hex constants uploaded to this device
