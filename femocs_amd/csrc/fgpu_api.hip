@@ -763,6 +763,7 @@ static Desc make_desc64(fgpu_sys *s, bool residual) {
     d.n_cells = m->n_cells;
     d.nb_cell = s->nb_cell;
     d.nb_dof = s->nb_dof;
+    d.dof_iter = s->dof_iter;
     d.cells = m->d_cells;
     d.X = m->d_X64;
     d.gptr = m->d_gptr;
@@ -833,6 +834,7 @@ static Desc make_desc32(fgpu_sys *s, bool coarse = false) {
     d.n_cells = m->n_cells;
     d.nb_cell = s->nb_cell;
     d.nb_dof = s->nb_dof;
+    d.dof_iter = s->dof_iter;
     d.cells = m->d_cells;
     d.X = m->d_X32;
     d.gptr = m->d_gptr;
@@ -876,6 +878,17 @@ static Desc make_desc32(fgpu_sys *s, bool coarse = false) {
     return d;
 }
 
+// dofs per thread of the system's per-dof kernels, and the partials that go with it
+static void set_dof_iter(fgpu_sys *s, int iter) {
+    hipStream_t st = s->ctx->stream;
+    s->dof_iter = iter;
+    s->nb_dof = padded_blocks(static_cast<fgpu_mesh *>(s->mesh)->n_dofs, kBlock * iter);
+    HIPCHECK(hipStreamSynchronize(st));
+    dfree(s->part);
+    s->part = dalloc<double>(2 * kPartRegions * (size_t)s->nb_dof);
+    HIPCHECK(hipMemsetAsync(s->part, 0, 2 * kPartRegions * (size_t)s->nb_dof * sizeof(double), st));
+}
+
 extern "C" int fgpu_sys_create(fgpu_mesh *m, fgpu_sys **out) {
     if (!m || !out) return FGPU_EINVAL;
     *out = nullptr;
@@ -887,7 +900,6 @@ extern "C" int fgpu_sys_create(fgpu_mesh *m, fgpu_sys **out) {
         HIPCHECK(hipSetDevice(m->ctx->device));
         const size_t n = m->n_dofs;
         s->nb_cell = padded_blocks(m->patches.n, s->ppb);
-        s->nb_dof = padded_blocks(m->n_dofs, kDofBlock);
         s->b = dalloc<double>(n); s->x = dalloc<double>(n); s->r = dalloc<double>(n); s->z = dalloc<double>(n);
         s->p = dalloc<double>(n); s->q = dalloc<double>(n);
         s->invd = dalloc<double>(n); s->diag = dalloc<double>(n); s->g = dalloc<double>(n); s->tmp = dalloc<double>(n);
@@ -897,10 +909,9 @@ extern "C" int fgpu_sys_create(fgpu_mesh *m, fgpu_sys **out) {
         s->d32 = dalloc<float>(n); s->invd32 = dalloc<float>(n);
         ensure_layout(s);
         s->scal = dalloc<double>(2 * kScal);
-        s->part = dalloc<double>(2 * kPartRegions * (size_t)s->nb_dof);
+        set_dof_iter(s, m->n_dofs <= kSmallDofs ? 1 : kDofIter);
         hipStream_t st = m->ctx->stream;
         HIPCHECK(hipMemsetAsync(s->scal, 0, 2 * kScal * sizeof(double), st));
-        HIPCHECK(hipMemsetAsync(s->part, 0, 2 * kPartRegions * (size_t)s->nb_dof * sizeof(double), st));
         HIPCHECK(hipMemsetAsync(s->b, 0, n * sizeof(double), st));
         HIPCHECK(hipMemsetAsync(s->x, 0, n * sizeof(double), st));
         HIPCHECK(hipMemsetAsync(s->g, 0, n * sizeof(double), st));
@@ -1706,8 +1717,9 @@ static int build_coarse(fgpu_sys *s, int shift) {
     s->cc64 = dalloc<double>(nc);
     launch_to_half(st, nc, ld, dA, cscale, s->cinv);
     HIPCHECK(hipMemsetAsync(s->cc, 0, nc * sizeof(float), st));
-    // the coarse partials of another aggregate size would stay in the sums over their region
-    HIPCHECK(hipMemsetAsync(s->part, 0, 2 * kPartRegions * (size_t)s->nb_dof * sizeof(double), st));
+    // fresh partials: the coarse ones of another aggregate size would stay in the sums over their
+    // region; a workgroup's dofs hold whole aggregates
+    set_dof_iter(s, n <= kSmallDofs && shift == 8 ? 1 : kDofIter);
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(st));
     dfree(dA);

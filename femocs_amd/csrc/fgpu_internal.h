@@ -16,6 +16,11 @@ namespace fgpu {
 constexpr int kBlock = 256;   // threads per workgroup (4 wave64)
 constexpr int kDofIter = 4;   // dofs per thread in the per-dof kernels
 constexpr int kDofBlock = kBlock * kDofIter;
+// dofs up to which a Q1 system's per-dof kernels run one dof per thread (256 per workgroup): with
+// four, 39k dofs are 38 workgroups on 256 CUs.  One against four, whole calls: 5k dofs 2.40 / 2.74
+// ms, 25k dofs 4.2 / 4.7 ms (mixed), 39k dofs (coupled step) 19.2 / 21.1 ms; 100k dofs gain 3 %, but
+// eight systems of 32k-96k dofs in one batch lose 4 % when all of them run it, 150k dofs lose 1 %
+constexpr int kSmallDofs = 49152;
 // coarse aggregates of the two-level preconditioner: 2^agg_shift consecutive internal dofs, a
 // multiple of kAggMin (one round of a dof workgroup) and at most its dofs
 constexpr int kAggMin = kBlock;
@@ -84,6 +89,7 @@ enum Scal : int {
 // launch's precision (double or float) where marked T.
 struct Desc {
     int n_dofs, n_cells, nb_cell, nb_dof;
+    int dof_iter;                 // dofs per thread of the per-dof kernels: 1 or kDofIter
     const int *cells;             // 8 per cell, lexicographic, internal dof ids
     const void *X;                // T4 coordinates per dof
     const int *gptr;              // dof i owns slot-buffer positions [gptr[i], gptr[i+1])
@@ -224,6 +230,7 @@ struct Sys {
     double *part = nullptr;       // 2 * kPartRegions*nb_dof
     double *ppq = nullptr;        // 2 x one p.q partial per patch (FP64 CG, FP32 CG)
     int nb_cell = 0, nb_dof = 0;
+    int dof_iter = kDofIter;      // dofs per thread of the per-dof kernels (sets nb_dof)
     int ppb = kPatchPerBlock;     // patches per element workgroup (tunable)
     int patch_gen = -1;           // mesh patch generation the slot buffers are sized for
     int diag_gen = -1;            // mesh coordinate generation the diagonal was computed for

@@ -488,20 +488,20 @@ template <class T, int CHUNK> __device__ __forceinline__ void gather_slots_wide(
     }
 }
 
-template <class T> __device__ __forceinline__ void gather_slots4(const Desc &d, int base, T (&q)[kDofIter]) {
+template <class T, int ITER> __device__ __forceinline__ void gather_slots4(const Desc &d, int base, T (&q)[ITER]) {
     const auto Ye = G(reinterpret_cast<const T *>(d.Ye));
     const auto gp = G(d.gptr);
-    int b[kDofIter], e[kDofIter];
+    int b[ITER], e[ITER];
 #pragma unroll
-    for (int m = 0; m < kDofIter; ++m) {
+    for (int m = 0; m < ITER; ++m) {
         const int i = base + threadIdx.x + m * kBlock;
         const int ii = i < d.n_dofs ? i : d.n_dofs - 1;
         b[m] = gp[ii];
         e[m] = gp[ii + 1];
     }
-    T v[kDofIter][4];
+    T v[ITER][4];
 #pragma unroll
-    for (int m = 0; m < kDofIter; ++m)
+    for (int m = 0; m < ITER; ++m)
 #pragma unroll
         for (int k = 0; k < 4; ++k) {
             const int idx = b[m] + k < e[m] ? b[m] + k : b[m];
@@ -509,7 +509,7 @@ template <class T> __device__ __forceinline__ void gather_slots4(const Desc &d, 
             v[m][k] = b[m] + k < e[m] ? y : (T)0;
         }
 #pragma unroll
-    for (int m = 0; m < kDofIter; ++m) {
+    for (int m = 0; m < ITER; ++m) {
         T s = 0;
 #pragma unroll
         for (int k = 0; k < 4; ++k) s += v[m][k];

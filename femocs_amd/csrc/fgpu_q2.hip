@@ -674,6 +674,7 @@ Desc q2_desc(fgpu_q2 *s) {
     d.n_dofs = s->n_dofs;
     d.n_cells = s->n_cells;
     d.nb_dof = s->nb_dof;
+    d.dof_iter = kDofIter;
     d.gptr = s->d_gptr;
     d.wide_slots = 1;             // vertex dofs own about two dozen slots each
     d.dmask = s->d_dmask;

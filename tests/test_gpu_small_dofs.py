@@ -1,0 +1,58 @@
+"""Per-dof kernels with one dof per thread (small systems) and four: solves on both sides of the
+limit and around whole workgroups agree with the oracle, alone and in one batch bit for bit, and a
+level of larger aggregates takes a small system back to four."""
+import numpy as np
+import pytest
+
+from femocs_amd import fgpu
+from femocs_amd import mesh as M
+from oracle import oracle as O
+
+pytestmark = pytest.mark.gpu
+MARKS = (8, 2, 4, 2)
+
+
+def _grid(nx, ny, nz):
+    X = np.stack(np.meshgrid(*[np.linspace(0.0, n, n) for n in (nx, ny, nz)], indexing="ij"), -1).reshape(-1, 3)
+    at = np.arange(nx * ny * nz).reshape(nx, ny, nz)
+    lex = np.stack([at[a:nx - 1 + a, b:ny - 1 + b, c:nz - 1 + c].reshape(-1) for c in (0, 1) for b in (0, 1)
+                    for a in (0, 1)], 1)
+    ucd = np.empty_like(lex)
+    ucd[:, M.UCD_TO_LEX] = lex
+    return X, ucd.astype(np.int32)
+
+
+def _system(ctx, X, ucd, agg):
+    s = fgpu.System(fgpu.Mesh(ctx, X, ucd, *MARKS))
+    s.reset()
+    s.add_dirichlet(2, 0.0)
+    s.add_neumann(8, None, -1.0)
+    s.apply_dirichlet()
+    if agg:
+        s.set_coarse(agg)
+    return s
+
+
+@pytest.mark.parametrize("precision, agg", [(fgpu.FGPU_FP64, 0), (fgpu.FGPU_MIXED, 0), (fgpu.FGPU_FP64, 256),
+                                            (fgpu.FGPU_MIXED, 256), (fgpu.FGPU_MIXED, 512), (fgpu.FGPU_MIXED, 1024)])
+def test_solves_around_the_limits(ctx, precision, agg):
+    # 256 and 257 dofs; 49152 (the last small size) and 49248
+    shapes = [(8, 8, 4), (257, 1 + 1, 2), (48, 32, 32), (48, 27, 38)]
+    o = fgpu.opts(tol=1e-12, precision=precision, inner_tol=0.01)
+    systems, alone = [], []
+    for shape in shapes:
+        X, ucd = _grid(*shape)
+        s = _system(ctx, X, ucd, agg)
+        s.fill_solution(0.0)
+        st = s.solve(o)
+        _, ref, it, _, _ = O.poisson_laplace(X, ucd, -1.0, tol=1e-13, relative=True)
+        assert st.iterations > 0 and it > 0
+        x = s.solution()
+        assert np.linalg.norm(x - ref) <= 1e-10 * np.linalg.norm(ref)
+        systems.append(s)
+        alone.append((st.iterations, x))
+    for s in systems:
+        s.fill_solution(0.0)
+    stats = ctx.solve_batch(systems, o)
+    for s, st, (it, x) in zip(systems, stats, alone):
+        assert st.iterations == it and np.array_equal(s.solution(), x)
