@@ -2004,6 +2004,8 @@ static SolveKind make_sets(const std::vector<fgpu_sys *> &sys, std::vector<std::
     return k;
 }
 
+static void wait_steps_of(fgpu_ctx *c, const std::vector<fgpu_sys *> &sys);
+
 // Starts the solves of a set of systems: scalars, x = g on constrained dofs, FP64 residual of
 // the lifted system and the first preconditioned residual (FP64), or the FP32 CG state
 // (mixed).  t: the set's uploaded tables.
@@ -2013,6 +2015,7 @@ static void start_solves(fgpu_ctx *c, const std::vector<fgpu_sys *> &sys, const 
     const bool mixed = k.mixed;
     const int max_it = std::max(0, o->max_it);
     const double delta = o->inner_tol > 0 && o->inner_tol < 1 ? o->inner_tol : 0.1;
+    wait_steps_of(c, sys);
     std::vector<double> h((size_t)2 * kScal * n, 0.0);
     for (int i = 0; i < n; ++i) {
         double *s64 = &h[(size_t)2 * kScal * i], *s32 = s64 + kScal;
@@ -2233,6 +2236,24 @@ struct fgpu_batch {
     hipEvent_t ev_ctx = nullptr;
 };
 
+// A member retired while a step is in flight is still a member of that step, whose kernels pass
+// it over only because its state says finished.  A new solve of it (in any batch, or alone)
+// therefore starts, on the context's stream, after the step.
+static void wait_steps_of(fgpu_ctx *c, const std::vector<fgpu_sys *> &sys) {
+    for (const fgpu_batch *b : c->in_flight)
+        for (fgpu_sys *s : sys)
+            if (std::find(b->pend_sys.begin(), b->pend_sys.end(), s) != b->pend_sys.end()) {
+                HIPCHECK(hipStreamWaitEvent(c->stream, b->pend_ev, 0));
+                break;
+            }
+}
+
+static void batch_landed(fgpu_batch *b) {
+    auto &f = b->ctx->in_flight;
+    f.erase(std::remove(f.begin(), f.end(), b), f.end());
+    b->pending = false;
+}
+
 static void batch_drop_graph(fgpu_batch *b) {
     if (b->exec) (void)hipGraphExecDestroy(b->exec);
     if (b->graph) (void)hipGraphDestroy(b->graph);
@@ -2273,6 +2294,7 @@ extern "C" void fgpu_batch_destroy(fgpu_batch *b) {
     (void)hipSetDevice(c->device);
     (void)hipStreamSynchronize(c->stream);
     if (b->st) (void)hipStreamSynchronize(b->st);
+    batch_landed(b);
     batch_drop_graph(b);
     for (auto *s : b->sys) s->batches--;
     if (b->st) (void)hipStreamDestroy(b->st);
@@ -2385,7 +2407,7 @@ extern "C" int fgpu_batch_step(fgpu_batch *b, int iterations, int *n_running) {
 static void batch_wait(fgpu_batch *b) {
     if (!b->pending) return;
     HIPCHECK(hipEventSynchronize(b->pend_ev));
-    b->pending = false;
+    batch_landed(b);
     b->last.clear();
     for (size_t i = 0; i < b->pend_sys.size(); ++i)
         if (std::find(b->joined.begin(), b->joined.end(), b->pend_sys[i]) == b->joined.end())
@@ -2415,6 +2437,7 @@ extern "C" int fgpu_batch_step_async(fgpu_batch *b, int iterations) {
         HIPCHECK(hipEventRecord(b->pend_ev, b->st));
         b->pend_sys = b->sys;
         b->joined.clear();
+        c->in_flight.push_back(b);
         b->pending = true;
         b->done_valid = false;
         return FGPU_OK;

@@ -308,6 +308,7 @@ struct fgpu_ctx {
     hipEvent_t stage_ev[kStage] = {};
     bool stage_busy[kStage] = {};
     int stage_next = 0;
+    std::vector<fgpu_batch *> in_flight;   // batches with an asynchronous step in flight
 };
 
 namespace fgpu {

@@ -240,7 +240,8 @@ int fgpu_batch_retire(fgpu_batch *batch, int max, fgpu_sys **out, fgpu_solve_sta
  * Between the two, the caller may retire the members a previous waited step finished and add
  * new ones (they join the next step); fgpu_batch_retire then uses the finished flags of the
  * last waited step.  Members that finished keep their results while later steps run (their
- * kernels skip finished systems).  One step in flight at a time (FGPU_EINVAL otherwise). */
+ * kernels skip finished systems), and a retired member may be solved again at once: that solve
+ * starts behind the step in flight.  One step in flight at a time (FGPU_EINVAL otherwise). */
 int fgpu_batch_step_async(fgpu_batch *batch, int iterations);
 int fgpu_batch_wait(fgpu_batch *batch, int *n_running);
 /* average duration (ms) of one launch of the element apply (which 0), the dof gather
