@@ -878,15 +878,24 @@ static Desc make_desc32(fgpu_sys *s, bool coarse = false) {
     return d;
 }
 
-// dofs per thread of the system's per-dof kernels, and the partials that go with it
+// dofs per thread of the system's per-dof kernels, and its partials, all zero (what another
+// aggregate size left would stay in the sums over their regions)
 static void set_dof_iter(fgpu_sys *s, int iter) {
     hipStream_t st = s->ctx->stream;
+    const int nb = padded_blocks(static_cast<fgpu_mesh *>(s->mesh)->n_dofs, kBlock * iter);
+    const size_t n = 2 * kPartRegions * (size_t)nb;
+    if (!s->part || nb != s->nb_dof) {
+        double *part = dalloc<double>(n);     // first: a failure leaves the system as it was
+        HIPCHECK(hipStreamSynchronize(st));
+        dfree(s->part);
+        s->part = part;
+        s->nb_dof = nb;
+    }
     s->dof_iter = iter;
-    s->nb_dof = padded_blocks(static_cast<fgpu_mesh *>(s->mesh)->n_dofs, kBlock * iter);
-    HIPCHECK(hipStreamSynchronize(st));
-    dfree(s->part);
-    s->part = dalloc<double>(2 * kPartRegions * (size_t)s->nb_dof);
-    HIPCHECK(hipMemsetAsync(s->part, 0, 2 * kPartRegions * (size_t)s->nb_dof * sizeof(double), st));
+    HIPCHECK(hipMemsetAsync(s->part, 0, n * sizeof(double), st));
+}
+static void set_dof_iter(fgpu_sys *s) {
+    set_dof_iter(s, static_cast<fgpu_mesh *>(s->mesh)->n_dofs <= kSmallDofs ? 1 : kDofIter);
 }
 
 extern "C" int fgpu_sys_create(fgpu_mesh *m, fgpu_sys **out) {
@@ -909,7 +918,7 @@ extern "C" int fgpu_sys_create(fgpu_mesh *m, fgpu_sys **out) {
         s->d32 = dalloc<float>(n); s->invd32 = dalloc<float>(n);
         ensure_layout(s);
         s->scal = dalloc<double>(2 * kScal);
-        set_dof_iter(s, m->n_dofs <= kSmallDofs ? 1 : kDofIter);
+        set_dof_iter(s);
         hipStream_t st = m->ctx->stream;
         HIPCHECK(hipMemsetAsync(s->scal, 0, 2 * kScal * sizeof(double), st));
         HIPCHECK(hipMemsetAsync(s->b, 0, n * sizeof(double), st));
@@ -1717,9 +1726,7 @@ static int build_coarse(fgpu_sys *s, int shift) {
     s->cc64 = dalloc<double>(nc);
     launch_to_half(st, nc, ld, dA, cscale, s->cinv);
     HIPCHECK(hipMemsetAsync(s->cc, 0, nc * sizeof(float), st));
-    // fresh partials: the coarse ones of another aggregate size would stay in the sums over their
-    // region; a workgroup's dofs hold whole aggregates
-    set_dof_iter(s, n <= kSmallDofs && shift == 8 ? 1 : kDofIter);
+    if (shift > 8) set_dof_iter(s, kDofIter);     // a workgroup's dofs hold whole aggregates
     HIPCHECK(hipGetLastError());
     HIPCHECK(hipStreamSynchronize(st));
     dfree(dA);
@@ -1740,6 +1747,7 @@ extern "C" int fgpu_sys_set_coarse(fgpu_sys *s, int enable, int *colors) {
         s->nc = 0;
         dfree(s->cinv);
         dfree(s->cc);
+        set_dof_iter(s);          // as a system that never had a level
         if (colors) *colors = 0;
         if (!enable) return FGPU_OK;
         if (!s->lifted) throw std::invalid_argument("apply the Dirichlet conditions before building the coarse level");

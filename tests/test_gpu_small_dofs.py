@@ -56,3 +56,23 @@ def test_solves_around_the_limits(ctx, precision, agg):
     stats = ctx.solve_batch(systems, o)
     for s, st, (it, x) in zip(systems, stats, alone):
         assert st.iterations == it and np.array_equal(s.solution(), x)
+
+
+@pytest.mark.parametrize("precision", [fgpu.FGPU_FP64, fgpu.FGPU_MIXED])
+@pytest.mark.parametrize("drop", ["off", "refused"])
+def test_dropped_level_leaves_no_trace(ctx, precision, drop):
+    """A small system whose level of larger aggregates was dropped gives the bits of one that
+    never had a level."""
+    X, ucd = _grid(24, 24, 24)
+    o = fgpu.opts(tol=1e-10, precision=precision, inner_tol=0.01)
+    out = []
+    for before in (False, True):
+        s = _system(ctx, X, ucd, 1024 if before else 0)
+        if before and drop == "off":
+            s.set_coarse(False)
+        elif before:
+            with pytest.raises(fgpu.FgpuError):
+                s.set_coarse(77)
+        s.fill_solution(0.0)
+        out.append((s.solve(o).iterations, s.solution()))
+    assert out[0][0] > 0 and out[0][0] == out[1][0] and np.array_equal(out[0][1], out[1][1])
