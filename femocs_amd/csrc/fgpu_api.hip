@@ -1695,8 +1695,8 @@ static int build_coarse(fgpu_sys *s, int shift) {
     HIPCHECK(hipGetLastError());
     // the inverse of an SPD matrix has a positive diagonal
     std::vector<double> dg(nc);
-    HIPCHECK(hipMemcpy2DAsync(dg.data(), sizeof(double), dA, (nc + 1) * sizeof(double), sizeof(double), nc,
-                              hipMemcpyDeviceToHost, st));
+    launch_diagonal(st, nc, dA, dV);
+    d2h(dg.data(), dV, nc, st);
     HIPCHECK(hipStreamSynchronize(st));
     dfree(dPi);
     dfree(dV);

@@ -31,6 +31,7 @@ void launch_coarse_sums(hipStream_t s, int n, const unsigned char *mask, const d
 int gj_block();
 void launch_gj_block(hipStream_t s, int n, int k, int bb, const double *A, double *B, double *Pi, double *V,
                      double *W);
+void launch_diagonal(hipStream_t s, int n, const double *a, double *out);
 void launch_to_half(hipStream_t s, int n, int ld, const double *a, double scale, _Float16 *out);
 void launch_enforce_dirichlet(hipStream_t s, int n, const unsigned char *mask, const double *g, double *x);
 void launch_lift(hipStream_t s, int n, const unsigned char *mask, const double *g, const double *Ag, const double *diag,

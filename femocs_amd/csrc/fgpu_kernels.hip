@@ -1747,6 +1747,14 @@ __global__ __launch_bounds__(256) void k_gj_update(int n, int k, int bb, const d
     B[e] = v;
 }
 
+// The diagonal of an n x n matrix, contiguous for the copy to the host.  A strided copy of 8-byte rows
+// gave other values for 45 rows while rocprofv3 traced the run (the coarse build then refused a sound
+// operator), and the same ones without it.
+__global__ __launch_bounds__(256) void k_diagonal(int n, const double *__restrict__ a, double *__restrict__ out) {
+    const int i = blockIdx.x * 256 + threadIdx.x;
+    if (i < n) out[i] = a[(size_t)i * n + i];
+}
+
 // out = a / scale in FP16 (scale a power of two: the division is exact before the rounding);
 // a: n x n, out: n rows of ld >= n entries, zero past n
 __global__ void k_to_half(int n, int ld, const double *__restrict__ a, double inv_scale, _Float16 *__restrict__ out) {
@@ -1773,6 +1781,9 @@ void launch_gj_block(hipStream_t s, int n, int k, int bb, const double *A, doubl
     hipLaunchKernelGGL(k_gj_pivot, dim3(1), dim3(256), 0, s, n, k, bb, A, Pi);
     hipLaunchKernelGGL(k_gj_panel, dim3((unsigned)((nb + 255) / 256)), dim3(256), 0, s, n, k, bb, A, Pi, V, W);
     hipLaunchKernelGGL(k_gj_update, dim3((unsigned)((e + 255) / 256)), dim3(256), 0, s, n, k, bb, A, Pi, V, W, B);
+}
+void launch_diagonal(hipStream_t s, int n, const double *a, double *out) {
+    if (n > 0) hipLaunchKernelGGL(k_diagonal, dim3((n + 255) / 256), dim3(256), 0, s, n, a, out);
 }
 void launch_to_half(hipStream_t s, int n, int ld, const double *a, double scale, _Float16 *out) {
     const size_t e = (size_t)n * ld;
