@@ -4,8 +4,8 @@ The matrix-free apply processes patches of consecutive cells per workgroup (thei
 staged in LDS); two knobs trade LDS reuse against parallelism and latency hiding:
 cells per patch (the elements-per-block of the element kernel) and patches handled in turn
 by one workgroup.  The best pair depends on the mesh size and on the precision, so it is
-measured on the system's own data: each candidate times the element apply plus the dof
-gather that consumes its output (the patch size changes the gather's work too).
+measured on the system's own data: each candidate times whole CG iterations (the patch size
+changes the vector kernel's slots too, and how the iteration's scalars are summed).
 
 The third knob is the unroll of a batched solve: how many CG iterations are captured in one
 hipGraph between two host convergence checks (more: fewer host round trips; fewer: less
@@ -25,16 +25,15 @@ PATCHES_PER_BLOCK = (1, 2, 4, 8)
 
 def autotune(system: fgpu.System, precision: int = fgpu.FGPU_MIXED, cells=CELLS, ppbs=PATCHES_PER_BLOCK,
              reps: int = 20, apply: bool = True):
-    """Returns (best (cells, ppb), table of {(cells, ppb): ms per apply + gather}) and, with
+    """Returns (best (cells, ppb), table of {(cells, ppb): ms per CG iteration}) and, with
     apply=True, leaves the system's mesh and the system set to the best pair."""
     mesh = system.mesh
     table = {}
     for c in cells:
         mesh.set_patch_cells(c)
-        gather = system.time_kernel(1, precision, reps)
         for ppb in ppbs:
             system.set_patches_per_block(ppb)
-            table[(c, ppb)] = system.time_kernel(0, precision, reps) + gather
+            table[(c, ppb)] = system.time_kernel(3, precision, reps)
     best = min(table, key=table.get)
     if apply:
         mesh.set_patch_cells(best[0])

@@ -1874,16 +1874,24 @@ static void cheb_steps(hipStream_t st, const Desc *D, const Desc *DC, const Batc
     }
 }
 
+// the element apply and the vector work of a CG iteration of every system of the set
+template <class T> static void cg_apply(hipStream_t st, const Desc *D, const BatchTabs &t, bool coef) {
+    launch_elem<T>(st, D, t.etab, t.ne, coef, false, true, S_BETA, sizeof(T) == 8 ? t.lds64 : t.lds32, t.affine32, t.fold,
+                   t.host(D));
+}
+template <class T> static void cg_vectors(hipStream_t st, const Desc *D, const BatchTabs &t) {
+    launch_cg_step<T>(st, D, t.dtab, t.nd, t.fold, t.host(D));
+}
+
 // one CG iteration of every system of the set; last: the state must be complete after it (the
 // scalar kernel that ends a folded iteration may be left out otherwise)
 template <class T>
 static void cg_iter(hipStream_t st, const Desc *D, const Desc *DC, const BatchTabs &t, int n, const SolveKind &k,
                     int reliable, bool last) {
     const Desc *one = t.host(D);
-    launch_elem<T>(st, D, t.etab, t.ne, k.coef, false, true, S_BETA, sizeof(T) == 8 ? t.lds64 : t.lds32, t.affine32, t.fold,
-                   one);
+    cg_apply<T>(st, D, t, k.coef);
     if (!t.fold) launch_scal_alpha(st, D, n, one);
-    launch_cg_step<T>(st, D, t.dtab, t.nd, t.fold, one);
+    cg_vectors<T>(st, D, t);
     if (sizeof(T) == 4) {
         launch_coarse(st, D, nullptr, t.ctab, t.nct, 0, one);
     } else {
@@ -2207,7 +2215,8 @@ static int solve_batch(fgpu_ctx *c, int n, fgpu_sys *const *systems, const fgpu_
 // ------------------------------------------------------------------------------------------
 // continuous batching: systems join and leave a running batch between steps
 // ------------------------------------------------------------------------------------------
-static double time_launches(fgpu_ctx *c, const Desc *D, const BatchTabs &t, bool coef, int which, int precision, int reps);
+static double time_launches(fgpu_ctx *c, const std::vector<fgpu_sys *> &sys, const fgpu_solve_opts *o, bool coef, int which,
+                            int reps);
 
 struct fgpu_batch {
     fgpu_ctx *ctx = nullptr;
@@ -2474,11 +2483,9 @@ extern "C" int fgpu_batch_time_kernel(fgpu_batch *b, int which, int reps, double
     return guarded(c, [&] {
         HIPCHECK(hipSetDevice(c->device));
         if (b->sys.empty()) throw std::invalid_argument("empty batch");
-        std::vector<std::vector<Desc>> sets;
-        make_sets(b->sys, sets, &b->o);
-        BatchTabs t = upload_batch(c, sets, b->sys);
-        const bool mixed = b->o.precision == FGPU_MIXED;
-        *avg_ms = time_launches(c, mixed ? t.sets[2] : t.sets[1], t, b->coef > 0, which, b->o.precision, reps);
+        // a step in flight uses the slot buffers too
+        if (b->pending) HIPCHECK(hipStreamWaitEvent(c->stream, b->pend_ev, 0));
+        *avg_ms = time_launches(c, b->sys, &b->o, b->coef > 0, which, reps);
         return FGPU_OK;
     });
 }
@@ -2537,33 +2544,71 @@ extern "C" int fgpu_sys_solve(fgpu_sys *s, const fgpu_solve_opts *o, fgpu_solve_
 
 // ------------------------------------------------------------------------------------------
 // kernel timing (benchmark helper): average duration of `reps` back-to-back launches of one
-// kernel of the solve, measured with HIP events on the context stream
+// kernel of a CG iteration, measured with HIP events on the context stream
 // ------------------------------------------------------------------------------------------
-// average duration of `reps` back-to-back launches of the element apply (which 0), the dof
-// gather (which 1) or the coarse product of the two-level FP32 CG (which 2) over descriptor
-// set D, HIP events on the context's stream
-static double time_launches(fgpu_ctx *c, const Desc *D, const BatchTabs &t, bool coef, int which, int precision, int reps) {
-    if (which == 2 && (precision != FGPU_MIXED || t.nct == 0)) throw std::invalid_argument("no coarse level in the batch");
+// average duration of `reps` back-to-back launches of the element apply (which 0), the vector work
+// (which 1) or the coarse product of the two-level FP32 CG (which 2), or of `reps` whole iterations
+// (which 3), HIP events on the context's stream.  The kernels and descriptors are those of the CG, in
+// an iteration that neither starts nor stops; what a later iteration reads (state, partials, vectors,
+// coarse corrections) is kept in copies, so that a running solve goes on undisturbed.
+static double time_launches(fgpu_ctx *c, const std::vector<fgpu_sys *> &sys, const fgpu_solve_opts *o, bool coef, int which,
+                            int reps) {
+    const bool mixed = o->precision == FGPU_MIXED;
+    hipStream_t st = c->stream;
+    struct Scratch {
+        std::vector<void *> p;
+        ~Scratch() {
+            for (void *q : p) (void)hipFree(q);
+        }
+        void *copy(hipStream_t st, const void *src, size_t bytes) {
+            p.push_back(dalloc<char>(bytes));
+            if (src) HIPCHECK(hipMemcpyAsync(p.back(), src, bytes, hipMemcpyDeviceToDevice, st));
+            return p.back();
+        }
+    } tmp;
+    std::vector<std::vector<Desc>> sets;
+    SolveKind kind = make_sets(sys, sets, o);
+    kind.coef = coef;
+    double h[kScal] = {};
+    h[S_ACTIVE] = h[S_GRUN] = 1.0;
+    h[S_THR2] = h[S_DELTA] = -1.0;             // never converged, never due for a reliable update
+    h[S_RRREF] = 1.0;
+    h[S_MAXIT] = 1e300;
+    const size_t word = mixed ? sizeof(float) : sizeof(double);
+    for (Desc &d : sets[mixed ? 2 : 0]) {
+        d.scal = static_cast<double *>(tmp.copy(st, nullptr, sizeof(h)));
+        stage_h2d(c, d.scal, h, sizeof(h));
+        d.part = static_cast<double *>(tmp.copy(st, d.part, kPartRegions * (size_t)d.nb_dof * sizeof(double)));
+        if (d.cc) d.cc = tmp.copy(st, d.cc, (size_t)d.nc * word);
+        if (which == 0 || which == 2) continue;
+        for (void **v : {&d.p, &d.x, &d.r, &d.zw}) *v = tmp.copy(st, *v, (size_t)d.n_dofs * word);
+    }
+    BatchTabs t = upload_batch(c, sets, sys);
+    if (which == 2 && (!mixed || t.nct == 0)) throw std::invalid_argument("no coarse level in the batch");
+    const Desc *D = t.sets[mixed ? 2 : 0];
     auto one = [&] {
         if (which == 2) {
-            launch_coarse(c->stream, D, nullptr, t.ctab, t.nct, 0);
+            launch_coarse(st, D, nullptr, t.ctab, t.nct, 0, t.host(D));
+        } else if (which == 3) {
+            if (mixed) cg_iter<float>(st, D, nullptr, t, (int)sys.size(), kind, 1, false);
+            else cg_iter<double>(st, D, nullptr, t, (int)sys.size(), kind, 0, false);
         } else if (which == 0) {
-            if (precision == FGPU_MIXED)
-                launch_elem<float>(c->stream, D, t.etab, t.ne, coef, false, false, S_BETA, t.lds32, t.affine32);
-            else launch_elem<double>(c->stream, D, t.etab, t.ne, coef, false, false, S_BETA, t.lds64);
+            if (mixed) cg_apply<float>(st, D, t, coef);
+            else cg_apply<double>(st, D, t, coef);
         } else {
-            if (precision == FGPU_MIXED) launch_gather_plain<float>(c->stream, D, t.dtab, t.nd, false);
-            else launch_gather_plain<double>(c->stream, D, t.dtab, t.nd, false);
+            if (mixed) cg_vectors<float>(st, D, t);
+            else cg_vectors<double>(st, D, t);
         }
     };
     one();
     hipEvent_t e0, e1;
     HIPCHECK(hipEventCreate(&e0));
     HIPCHECK(hipEventCreate(&e1));
-    HIPCHECK(hipEventRecord(e0, c->stream));
+    HIPCHECK(hipEventRecord(e0, st));
     for (int i = 0; i < reps; ++i) one();
-    HIPCHECK(hipEventRecord(e1, c->stream));
+    HIPCHECK(hipEventRecord(e1, st));
     HIPCHECK(hipEventSynchronize(e1));
+    HIPCHECK(hipGetLastError());
     float ms = 0;
     HIPCHECK(hipEventElapsedTime(&ms, e0, e1));
     (void)hipEventDestroy(e0);
@@ -2577,10 +2622,10 @@ extern "C" int fgpu_sys_time_kernel(fgpu_sys *s, int which, int precision, int r
         fgpu_ctx *c = s->ctx;
         HIPCHECK(hipSetDevice(c->device));
         ensure_diag(s);
-        Desc d = precision == FGPU_MIXED ? make_desc32(s) : make_desc64(s, true);
-        // inputs: the current z / x vectors; outputs: the slot buffer and q
-        BatchTabs t = upload_batch(c, {{d}}, {s});
-        *avg_ms = time_launches(c, t.sets[0], t, s->have_coef, which, precision, reps);
+        fgpu_solve_opts o{};
+        o.precision = precision;
+        o.precond = FGPU_PC_JACOBI;
+        *avg_ms = time_launches(c, {s}, &o, s->have_coef, which, reps);
         return FGPU_OK;
     });
 }

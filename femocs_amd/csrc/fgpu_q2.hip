@@ -1067,12 +1067,12 @@ extern "C" int fgpu_q2_time_apply(fgpu_q2 *s, int reps, double *avg_ms) {
     return q2_guarded(s->ctx, [&] {
         Q2CHECK(hipSetDevice(s->ctx->device));
         hipStream_t st = s->ctx->stream;
-        q2_apply(s, s->z, s->p, false, false);
+        q2_apply(s, s->z, s->p, false, false, s->ppq);
         hipEvent_t e0, e1;
         Q2CHECK(hipEventCreate(&e0));
         Q2CHECK(hipEventCreate(&e1));
         Q2CHECK(hipEventRecord(e0, st));
-        for (int i = 0; i < reps; ++i) q2_apply(s, s->z, s->p, false, false);
+        for (int i = 0; i < reps; ++i) q2_apply(s, s->z, s->p, false, false, s->ppq);
         Q2CHECK(hipEventRecord(e1, st));
         Q2CHECK(hipEventSynchronize(e1));
         float ms = 0;

@@ -244,10 +244,10 @@ int fgpu_batch_retire(fgpu_batch *batch, int max, fgpu_sys **out, fgpu_solve_sta
  * starts behind the step in flight.  One step in flight at a time (FGPU_EINVAL otherwise). */
 int fgpu_batch_step_async(fgpu_batch *batch, int iterations);
 int fgpu_batch_wait(fgpu_batch *batch, int *n_running);
-/* average duration (ms) of one launch of the element apply (which 0), the dof gather
- * (which 1) or the coarse product of the two-level preconditioner (which 2, mixed batches
- * with a coarse level) over all members, in the batch's precision; for measurement, no
- * counterpart in the reference.  Overwrites the members' slot buffers and coarse corrections. */
+/* average duration (ms) of one launch of a CG iteration's element apply (which 0), vector work
+ * (which 1) or coarse product of the two-level preconditioner (which 2, mixed batches with a
+ * coarse level), or of one whole iteration (which 3), over all members, in the batch's precision;
+ * for measurement, no counterpart in the reference.  Running solves go on undisturbed. */
 int fgpu_batch_time_kernel(fgpu_batch *batch, int which, int reps, double *avg_ms);
 /* ---- transfer to atoms (Interpolator, InterpolatorCells, SolutionReader) ---------------
  * An interpolator holds the tet mesh, its Tethex hexes (4 per tet, hex 4t+k around vertex k,
@@ -393,9 +393,9 @@ int fgpu_sys_minmax(fgpu_sys *sys, double *min, double *max);
 int fgpu_sys_solution_grad(fgpu_sys *sys, double *grad);
 
 /* Benchmark helper, no counterpart in the reference: average duration in ms of `reps`
- * back-to-back launches of one kernel of the CG step on this system's data (which = 0: the
- * element apply, 1: the dof gather, in the given precision), timed with HIP events on the
- * context stream. */
+ * back-to-back launches of a CG iteration's kernels on this system's data, in the given precision,
+ * with the Jacobi preconditioner and the coarse level if there is one (which as in
+ * fgpu_batch_time_kernel), timed with HIP events on the context stream. */
 int fgpu_sys_time_kernel(fgpu_sys *sys, int which, int precision, int reps, double *avg_ms);
 
 /* ---- the reference's tet -> 4-hex split (Tethex Mesh::convert_3D, src/Tethex.cpp:965-1169) ----
