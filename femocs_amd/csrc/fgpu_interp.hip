@@ -28,6 +28,8 @@ using namespace fgpu;
 // contiguous, so the records of a descent share cache lines.
 //   find: box of the subtree's cells (leaf: of its cell)
 //   near: box of the subtree's centroids (leaf: its centroid, three doubles in the place of the box)
+// The arrays that they are written from (child pairs, boxes, leaf order: 84 bytes a cell) are
+// temporaries of the build; the faces keep those that the centroid lookup walks.
 struct __align__(32) TreeNode {
     float b[6];
     int cell;       // the leaf's cell, -1 for an internal node
@@ -43,9 +45,7 @@ struct fgpu_interp {
     // device tables
     double *xyz = nullptr, *det0 = nullptr, *det = nullptr, *cen = nullptr;
     int *tets = nullptr, *c10 = nullptr, *hexes = nullptr, *marker = nullptr;
-    int *child = nullptr, *prim = nullptr;
     TreeNode *find = nullptr;        // preorder records of the tet tree (find, then near)
-    float *box = nullptr, *cbox = nullptr, *leafbox = nullptr;
     int *n2c_ptr = nullptr, *n2c = nullptr, *vor_ptr = nullptr, *vor = nullptr;
     double *sol = nullptr;                  // 5 per node: vector xyz, scalar1, scalar2
     double *un = nullptr;                   // the potential per node (extraction; on demand)
@@ -76,7 +76,7 @@ struct fgpu_interp {
     TreeNode *tri_find = nullptr;    // the same of the face tree
     int *tri_nbr_ptr = nullptr, *tri_nbr = nullptr;   // face neighbour lists (LinearTriangles)
     int *tri2tet = nullptr, *quad2hex = nullptr;       // the two tets of a face, hexes of a quad
-    float *tri_box = nullptr, *tri_cbox = nullptr, *tri_leafbox = nullptr;
+    float *tri_cbox = nullptr;
     // quadrangles: nodes, 6-node faces, centroids and their tree
     Bvh QB;
     double *quad_cen = nullptr;
@@ -1014,7 +1014,7 @@ void free_triangles(fgpu_interp *ip) {
     for (int **p : {&ip->tri_child, &ip->tri_prim, &ip->tri_nodes, &ip->quad_nodes, &ip->tri6, &ip->quad_child,
                     &ip->quad_prim, &ip->tri_nbr_ptr, &ip->tri_nbr, &ip->tri2tet, &ip->quad2hex})
         release(*p);
-    for (float **p : {&ip->tri_box, &ip->tri_cbox, &ip->tri_leafbox, &ip->quad_cbox}) release(*p);
+    for (float **p : {&ip->tri_cbox, &ip->quad_cbox}) release(*p);
     release(ip->tri_find);
     ip->T = LinTriHost{};
     ip->TB = Bvh{};
@@ -1023,12 +1023,11 @@ void free_triangles(fgpu_interp *ip) {
 
 void free_interp(fgpu_interp *ip) {
     for (double **p : {&ip->xyz, &ip->det0, &ip->det, &ip->cen, &ip->sol, &ip->un, &ip->pts, &ip->out}) release(*p);
-    for (int **p : {&ip->tets, &ip->c10, &ip->hexes, &ip->marker, &ip->child, &ip->prim, &ip->n2c_ptr, &ip->n2c,
+    for (int **p : {&ip->tets, &ip->c10, &ip->hexes, &ip->marker, &ip->n2c_ptr, &ip->n2c,
                     &ip->vor_ptr, &ip->vor, &ip->node_idof, &ip->tet, &ip->cells, &ip->cells2, &ip->d_region_hex,
                     &ip->sc_icell,
                     &ip->d_hex_cell, &ip->d_nbr_ptr, &ip->d_nbr})
         release(*p);
-    for (float **p : {&ip->box, &ip->cbox, &ip->leafbox}) release(*p);
     release(ip->find);
     release(ip->cand);
     release(ip->cand2);
@@ -1065,7 +1064,7 @@ __global__ __launch_bounds__(256) void k_point_codes(int n, const double *__rest
 
 // the order in which the point searches take the n points of ip->pts (their Morton order in the
 // tree's root box), or nullptr where sorting does not pay (few points, a one-leaf tree)
-const int *point_order(fgpu_interp *ip, int n, int n_leaves, const float *root_box) {
+const int *point_order(fgpu_interp *ip, int n, int n_leaves, const TreeNode *tree) {
     if (n < 2048 || n_leaves < 2) return nullptr;
     hipStream_t st = ip->ctx->stream;
     if ((size_t)n > ip->sort_cap) {
@@ -1087,7 +1086,7 @@ const int *point_order(fgpu_interp *ip, int n, int n_leaves, const float *root_b
         IPCHECK(hipMalloc(&ip->stmp, bytes));
         ip->stmp_bytes = bytes;
     }
-    hipLaunchKernelGGL(k_point_codes, dim3(grid(n)), dim3(256), 0, st, n, ip->pts, root_box, ip->skey, ip->sidx);
+    hipLaunchKernelGGL(k_point_codes, dim3(grid(n)), dim3(256), 0, st, n, ip->pts, tree->b, ip->skey, ip->sidx);
     IPCHECK(hipcub::DeviceRadixSort::SortPairs(ip->stmp, bytes, ip->skey, ip->skey2, ip->sidx, ip->sperm, n, 0, 63, st));
     return ip->sperm;
 }
@@ -1112,32 +1111,9 @@ void launch_candidates(hipStream_t s, int n, const double *pts, int n_leaves, co
 }
 
 void tet_candidates(fgpu_interp *ip, int n, int4 *cand, int *lst = nullptr) {
-    const int *perm = point_order(ip, n, ip->B.n_leaves, ip->box);
+    const int *perm = point_order(ip, n, ip->B.n_leaves, ip->find);
     launch_candidates(ip->ctx->stream, n, ip->pts, ip->B.n_leaves, ip->find, TetCells{ip->det0, ip->det, ip->marker}, ip->cen,
                       cand, lst, perm);
-}
-
-// the preorder records of a tree of nl leaves (device arrays) in a new array: 2 nl - 1 find
-// records, then as many near records
-TreeNode *tree_records(hipStream_t s, int nl, const int *child, const float *box, const float *cbox, const float *leafbox,
-                       const int *prim, const double *cen) {
-    const int ni = std::max(nl - 1, 0), nn = std::max(2 * nl - 1, 0);
-    TreeNode *rec = nullptr;
-    int *par = nullptr;
-    IPCHECK(hipMalloc(&rec, std::max<size_t>(2 * (size_t)nn, 1) * sizeof(TreeNode)));
-    if (nl <= 0) return rec;
-    hipError_t e = hipMalloc(&par, (size_t)nn * sizeof(int));
-    if (e == hipSuccess) {
-        if (ni > 0) hipLaunchKernelGGL(kb_parents, dim3(grid(ni)), dim3(256), 0, s, ni, child, par);
-        hipLaunchKernelGGL(kb_preorder, dim3(grid(nn)), dim3(256), 0, s, nl, child, par, box, cbox, leafbox, prim, cen, rec,
-                           rec + nn);
-        e = hipGetLastError();
-        if (e == hipSuccess) e = hipStreamSynchronize(s);
-        (void)hipFree(par);
-    }
-    if (e != hipSuccess) (void)hipFree(rec);
-    IPCHECK(e);
-    return rec;
 }
 
 // the chained guess over the located points (ip->pts, n of them) into ip->tet, in the
@@ -1304,18 +1280,16 @@ extern "C" int fgpu_interp_create_ex(fgpu_ctx *c, int n_nodes, const double *xyz
             ip->cen = upload(ip->L.centroid.data(), ip->L.centroid.size(), s);
             ip->marker = upload(ip->L.marker.data(), ip->L.marker.size(), s);
             ip->c10 = upload(c10.data(), c10.size(), s);
-            ip->child = upload(ip->B.child.data(), ip->B.child.size(), s);
-            ip->box = upload(ip->B.box.data(), ip->B.box.size(), s);
-            ip->cbox = upload(ip->B.cbox.data(), ip->B.cbox.size(), s);
-            ip->leafbox = upload(ip->B.leafbox.data(), ip->B.leafbox.size(), s);
-            ip->prim = upload(ip->B.prim.data(), ip->B.prim.size(), s);
             ip->n2c_ptr = upload(nptr.data(), nptr.size(), s);
             ip->n2c = upload(n2c.data(), n2c.size(), s);
             ip->vor_ptr = upload(vptr.data(), vptr.size(), s);
             ip->vor = upload(vor.data(), vor.size(), s);
+            BArena tmp(96 * (size_t)n_tets + (1 << 16));
+            tree_records(s, ip->B.n_leaves, to_arena(ip->B.child, s, tmp), to_arena(ip->B.box, s, tmp),
+                         to_arena(ip->B.cbox, s, tmp), to_arena(ip->B.leafbox, s, tmp), to_arena(ip->B.prim, s, tmp), ip->cen,
+                         tmp, ip->find);
             IPCHECK(hipStreamSynchronize(s));   // the host vectors are read until the copies end
         }
-        ip->find = tree_records(s, ip->B.n_leaves, ip->child, ip->box, ip->cbox, ip->leafbox, ip->prim, ip->cen);
         // the nodal solution starts at the empty value everywhere (filled on the device)
         IPCHECK(hipMalloc(&ip->sol, 5 * (size_t)n_nodes * sizeof(double)));
         launch_set_const(s, 5 * n_nodes, empty_value, ip->sol);
@@ -1358,7 +1332,7 @@ extern "C" int fgpu_interp_digest(fgpu_interp *ip, int n, unsigned long long *ou
         IPCHECK(hipSetDevice(ip->ctx->device));
         hipStream_t st = ip->ctx->stream;
         ensure_host_tets(ip);
-        const size_t nt = ip->n_tets, ni = nt > 0 ? nt - 1 : 0;
+        const size_t nt = ip->n_tets, nn = nt > 0 ? 2 * nt - 1 : 0;   // nn: nodes of the tree
         const LinTetHost &L = ip->L;
         int k = 0;
         out[k++] = fnv_host(L.det0);
@@ -1373,11 +1347,8 @@ extern "C" int fgpu_interp_digest(fgpu_interp *ip, int n, unsigned long long *ou
         out[k++] = fnv_device(ip->marker, nt, st);
         out[k++] = fnv_device(ip->d_nbr_ptr, nt + 1, st);
         out[k++] = fnv_device(ip->d_nbr, (size_t)ip->n_nbr, st);
-        out[k++] = fnv_device(ip->child, 2 * ni, st);
-        out[k++] = fnv_device(ip->box, 6 * ni, st);
-        out[k++] = fnv_device(ip->cbox, 6 * ni, st);
-        out[k++] = fnv_device(ip->leafbox, 6 * nt, st);
-        out[k++] = fnv_device(ip->prim, nt, st);
+        out[k++] = fnv_device(ip->find, nn, st);
+        out[k++] = fnv_device(ip->find + nn, nn, st);
         out[k++] = fnv_device(ip->c10, 10 * nt, st);
         out[k++] = fnv_device(ip->n2c_ptr, (size_t)ip->n_nodes + 1, st);
         out[k++] = fnv_device(ip->n2c, (size_t)ip->n_n2c, st);
@@ -1938,11 +1909,10 @@ extern "C" int fgpu_interp_set_triangles(fgpu_interp *ip, int n_tris, const int 
         ip->tri_nodes = upload(ip->T.tris.data(), ip->T.tris.size(), s);
         ip->tri_child = upload(ip->TB.child.data(), ip->TB.child.size(), s);
         ip->tri_prim = upload(ip->TB.prim.data(), ip->TB.prim.size(), s);
-        ip->tri_box = upload(ip->TB.box.data(), ip->TB.box.size(), s);
         ip->tri_cbox = upload(ip->TB.cbox.data(), ip->TB.cbox.size(), s);
-        ip->tri_leafbox = upload(ip->TB.leafbox.data(), ip->TB.leafbox.size(), s);
-        ip->tri_find = tree_records(s, ip->TB.n_leaves, ip->tri_child, ip->tri_box, ip->tri_cbox, ip->tri_leafbox,
-                                    ip->tri_prim, ip->tri_cen);
+        BArena tmp(64 * (size_t)n_tris + (1 << 16));
+        tree_records(s, ip->TB.n_leaves, ip->tri_child, to_arena(ip->TB.box, s, tmp), ip->tri_cbox,
+                     to_arena(ip->TB.leafbox, s, tmp), ip->tri_prim, ip->tri_cen, tmp, ip->tri_find);
         ip->tri_nbr_ptr = upload(ip->T.nbr_ptr.data(), ip->T.nbr_ptr.size(), s);
         ip->tri_nbr = upload(ip->T.nbr.data(), ip->T.nbr.size(), s);
         ip->tri2tet = upload(ip->T.tri2tet.data(), ip->T.tri2tet.size(), s);
@@ -1969,7 +1939,7 @@ static bool device_surface(fgpu_interp *ip, int n, int *cells, double *out, int 
     IPCHECK(hipMemsetAsync(ip->chain_flag, 0, sizeof(int), st));
     tet_candidates(ip, n, ip->cand);
     if (locate) {
-        const int *perm = point_order(ip, n, ip->TB.n_leaves, ip->tri_box);
+        const int *perm = point_order(ip, n, ip->TB.n_leaves, ip->tri_find);
         launch_candidates(st, n, ip->pts, ip->TB.n_leaves, ip->tri_find, TriCells{ip->tri_tab}, ip->tri_cen, ip->cand2,
                           ip->chain_lst, perm);
         // the first guess: |-1| as a face, or |-1| / 3 from the quadrangle numbering

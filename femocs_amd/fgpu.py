@@ -19,7 +19,7 @@ FGPU_IMPORT_HOST = 1
 FGPU_MESH_DIGEST_TABLES = 32
 FGPU_INTERP_HOST = 1
 FGPU_INTERP_HOST_CHAIN = 2
-FGPU_INTERP_DIGEST_TABLES = 23
+FGPU_INTERP_DIGEST_TABLES = 20
 BID_COPPER_SURFACE, BID_VACUUM_TOP, BID_COPPER_BOTTOM, BID_SIDES = 2, 8, 7, 4
 
 _lib = None

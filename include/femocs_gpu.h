@@ -281,7 +281,7 @@ int fgpu_interp_create_ex(fgpu_ctx *ctx, int n_nodes, const double *xyz, const i
 /* 64-bit FNV-1a hashes of every interpolator table (host copy of the tet tables, device
  * tables, the smoothing decay), n >= FGPU_INTERP_DIGEST_TABLES.  No counterpart in the
  * reference. */
-#define FGPU_INTERP_DIGEST_TABLES 23
+#define FGPU_INTERP_DIGEST_TABLES 20
 int fgpu_interp_digest(fgpu_interp *interp, int n, unsigned long long *out);
 void fgpu_interp_destroy(fgpu_interp *interp);
 /* Interpolator::extract_solution(PoissonSolver&, smoothen) (src/Interpolator.cpp:142-190): from
