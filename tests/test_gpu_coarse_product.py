@@ -7,25 +7,12 @@ import numpy as np
 import pytest
 import scipy.sparse as sp
 
+from box_grid import box_grid
 from femocs_amd import fgpu
-from femocs_amd import mesh as M
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 MARKS = (8, 2, 4, 2)
-
-
-def _grid(nx, ny, nz):
-    """(nx - 1)(ny - 1)(nz - 1) hexes of a jittered box grid, UCD order."""
-    X = np.stack(np.meshgrid(*[np.linspace(0.0, n, n) for n in (nx, ny, nz)], indexing="ij"), -1).reshape(-1, 3)
-    inner = np.all((X > 0) & (X < [nx, ny, nz]), axis=1)
-    X[inner] += np.random.default_rng(3).uniform(-0.2, 0.2, (inner.sum(), 3))
-    at = np.arange(nx * ny * nz).reshape(nx, ny, nz)
-    lex = np.stack([at[a:nx - 1 + a, b:ny - 1 + b, c:nz - 1 + c].reshape(-1) for c in (0, 1) for b in (0, 1)
-                    for a in (0, 1)], 1)
-    ucd = np.empty_like(lex)
-    ucd[:, M.UCD_TO_LEX] = lex
-    return X, ucd.astype(np.int32)
 
 
 def _system(ctx, X, ucd):
@@ -37,14 +24,19 @@ def _system(ctx, X, ucd):
     return s
 
 
-# aggregates: 1, 12 (a row of 16 entries), 512 and 513 (one and two waves), 1024 and 1025 (two and
-# four waves, two octets for some lanes of the last)
+# aggregates: 1; 5, 6 and 7 (the last group of four rows holds 1, 2 and 3); 12 (a row of 16 entries);
+# 512 and 513 (one and two waves a group, 513 ends in a group of one row), 528; 1024 and 1025 (two and
+# four waves, two octets for some lanes of the last), 1040; larger aggregates, 257 of 512 dofs and 129
+# of 1024 in a cut group
 @pytest.mark.parametrize("shape, agg, nc", [((6, 7, 5), 256, 1), ((14, 15, 14), 256, 12), ((64, 64, 32), 256, 512),
+                                            ((9, 10, 12), 256, 5), ((9, 11, 13), 256, 6), ((10, 12, 13), 256, 7),
+                                            ((41, 50, 64), 256, 513), ((41, 79, 81), 256, 1025),
+                                            ((41, 50, 64), 512, 257), ((41, 50, 64), 1024, 129),
                                             ((64, 64, 33), 256, 528), ((64, 64, 64), 256, 1024),
                                             ((65, 64, 64), 256, 1040), ((64, 64, 33), 512, 264),
                                             ((64, 64, 33), 1024, 132)])
 def test_coarse_product_rows(ctx, shape, agg, nc):
-    X, ucd = _grid(*shape)
+    X, ucd = box_grid(*shape, jitter=0.2)
     s = _system(ctx, X, ucd)
     s.set_coarse(agg)
     block, einv = s.coarse()
@@ -71,7 +63,7 @@ def test_coarse_product_rows(ctx, shape, agg, nc):
 @pytest.mark.parametrize("precision", [fgpu.FGPU_FP64, fgpu.FGPU_MIXED])
 def test_coarse_level_rebuilt_at_another_size(ctx, precision):
     """The partial sums of the smaller aggregates must not stay in the larger ones' r.z."""
-    X, ucd = _grid(24, 24, 24)
+    X, ucd = box_grid(24, 24, 24, jitter=0.2)
     o = fgpu.opts(tol=1e-10, precision=precision, inner_tol=0.01)
     out = []
     for sizes in ((1024,), (256, 1024)):

@@ -59,3 +59,27 @@ def test_lanes_per_point_find_the_same_cells(ctx, small_mesh):
     one = ip.points(pts, 1)[0]
     for n in (131072, 32768, 777):
         assert np.array_equal(ip.points(pts[:n], 1)[0], one[:n])
+
+
+@pytest.mark.parametrize("rank", [1, 3])
+def test_lanes_per_point_find_the_same_faces(ctx, small_mesh, rank):
+    """The surface search (faces and the tets behind them) at one, 8 and 16 lanes a point: the chain
+    of a call's first points is that of a shorter call, also with atoms on face vertices and edges,
+    which lie in several faces."""
+    tip = small_mesh
+    tris, t2t = tip.surface_triangles()
+    ip = interp.Interpolator(ctx, tip, interp.TYPES_VACUUM)
+    ip.set_triangles(tris, t2t, tip.surface_quads(tris))
+    rng = np.random.default_rng(21)
+    ip.set_nodal(rng.standard_normal((len(tip.nodes), 5)))
+    n = 131073
+    w = rng.dirichlet(np.ones(3), n)
+    w[::5] = np.eye(3)[rng.integers(0, 3, len(w[::5]))]              # vertices
+    w[1::5, 0], w[1::5, 1], w[1::5, 2] = 0.5, 0.5, 0.0               # edge centres
+    pts = np.einsum("nk,nkd->nd", w, tip.nodes[tris[rng.integers(0, len(tris), n)]])
+    pts[2::5] += rng.normal(0.0, 0.3, pts[2::5].shape)               # off the surface
+    one, val = ip.surface_points(pts, rank)
+    assert (one < 0).any() and (one > 0).any()
+    for m in (131072, 32769, 32768, 777):
+        cells, out = ip.surface_points(pts[:m], rank)
+        assert np.array_equal(cells, one[:m]) and np.array_equal(out, val[:m])

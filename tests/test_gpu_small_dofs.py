@@ -4,22 +4,12 @@ level of larger aggregates takes a small system back to four."""
 import numpy as np
 import pytest
 
+from box_grid import box_grid
 from femocs_amd import fgpu
-from femocs_amd import mesh as M
 from oracle import oracle as O
 
 pytestmark = pytest.mark.gpu
 MARKS = (8, 2, 4, 2)
-
-
-def _grid(nx, ny, nz):
-    X = np.stack(np.meshgrid(*[np.linspace(0.0, n, n) for n in (nx, ny, nz)], indexing="ij"), -1).reshape(-1, 3)
-    at = np.arange(nx * ny * nz).reshape(nx, ny, nz)
-    lex = np.stack([at[a:nx - 1 + a, b:ny - 1 + b, c:nz - 1 + c].reshape(-1) for c in (0, 1) for b in (0, 1)
-                    for a in (0, 1)], 1)
-    ucd = np.empty_like(lex)
-    ucd[:, M.UCD_TO_LEX] = lex
-    return X, ucd.astype(np.int32)
 
 
 def _system(ctx, X, ucd, agg):
@@ -36,12 +26,13 @@ def _system(ctx, X, ucd, agg):
 @pytest.mark.parametrize("precision, agg", [(fgpu.FGPU_FP64, 0), (fgpu.FGPU_MIXED, 0), (fgpu.FGPU_FP64, 256),
                                             (fgpu.FGPU_MIXED, 256), (fgpu.FGPU_MIXED, 512), (fgpu.FGPU_MIXED, 1024)])
 def test_solves_around_the_limits(ctx, precision, agg):
-    # 256 and 257 dofs; 49152 (the last small size) and 49248
-    shapes = [(8, 8, 4), (257, 1 + 1, 2), (48, 32, 32), (48, 27, 38)]
+    # 256 dofs (one workgroup), 258, 1028 (four workgroups and 4 dofs); 49152 (the last small size)
+    # and 49248
+    shapes = [(8, 8, 4), (2, 3, 43), (257, 2, 2), (48, 32, 32), (48, 27, 38)]
     o = fgpu.opts(tol=1e-12, precision=precision, inner_tol=0.01)
     systems, alone = [], []
     for shape in shapes:
-        X, ucd = _grid(*shape)
+        X, ucd = box_grid(*shape)
         s = _system(ctx, X, ucd, agg)
         s.fill_solution(0.0)
         st = s.solve(o)
@@ -63,7 +54,7 @@ def test_solves_around_the_limits(ctx, precision, agg):
 def test_dropped_level_leaves_no_trace(ctx, precision, drop):
     """A small system whose level of larger aggregates was dropped gives the bits of one that
     never had a level."""
-    X, ucd = _grid(24, 24, 24)
+    X, ucd = box_grid(24, 24, 24)
     o = fgpu.opts(tol=1e-10, precision=precision, inner_tol=0.01)
     out = []
     for before in (False, True):
