@@ -786,7 +786,6 @@ static Desc make_desc64(fgpu_sys *s, bool residual) {
     d.Ye = s->Ye;
     d.q = s->q;
     d.p = s->p;
-    d.z = s->z;
     d.x = s->x;
     d.r = s->r;
     d.zw = s->z;
@@ -857,7 +856,6 @@ static Desc make_desc32(fgpu_sys *s, bool coarse = false) {
     d.Ye = s->Ye32;
     d.q = s->q32;
     d.p = s->p32;
-    d.z = s->z32;
     d.x = s->d32;
     d.r = s->r32;
     d.zw = s->z32;

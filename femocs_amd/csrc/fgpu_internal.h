@@ -105,8 +105,7 @@ struct Desc {
     void *Ye;                     // T: element outputs, dof-major (see gptr/spos)
     void *q;                      // T: gathered A u (plain products)
     void *p;                      // T: search direction
-    const void *z;                // T: preconditioned residual
-    void *x, *r, *zw;             // T: iterate, residual, preconditioned residual (written)
+    void *x, *r, *zw;             // T: iterate, residual, preconditioned residual
     const void *invdiag;          // T: 1/diag, 0 on constrained dofs
     const double *b;              // FP64 rhs (residual mode)
     double *scal;                 // kScal doubles

@@ -6,9 +6,10 @@
 //             (sum-factorised reference gradients, per-point metric, transposed sum
 //             factorisation), per-node sums in LDS (FP64: in a fixed order; FP32: exact
 //             fixed-point sums), one store per (node, patch) into the dof-major slot buffer
-//   k_gather  one thread per dof: add the dof's slots in ascending order, fused with the
-//             CG vector work of that step and a block reduction into per-block partials,
-//             which a one-block-per-system scalar kernel sums in block order
+//   per-dof kernels (fgpu_cg.inc): one thread adds a dof's slots in ascending order, fused with
+//             the CG vector work of that step and a block reduction into per-block partials,
+//             which are summed in block order by a one-block-per-system scalar kernel or, for
+//             small systems, by every workgroup of the next launch
 // No floating-point atomics anywhere, so a system gives bit-identical results whatever
 // other systems share the launch.  Every kernel walks a block table (system, local block),
 // which is how one launch serves a batch of meshes of any sizes.
@@ -371,7 +372,6 @@ __device__ __forceinline__ double fold_alpha(const Desc &d, double share, bool l
     return alpha;
 }
 
-// the dof's element outputs sit contiguously in the slot buffer, in ascending cell order
 // Global-memory views of the descriptor's pointers: loads and stores through them are
 // global_load/global_store (scalar base + vector offset) instead of flat accesses, which also
 // count against the LDS counter and would make every LDS wait wait for them too.
@@ -414,14 +414,9 @@ template <class T> __device__ __forceinline__ T coarse_term(const Desc &d, int i
     return c * keep;
 }
 
-// Slot sums of the kDofIter dofs a thread of a dof workgroup handles (base + threadIdx.x +
-// m * kBlock), each in ascending slot order.  The slot offsets of all of them are loaded
-// first, then up to four slots each in one wave (indices clamped into the dof's own range, the
-// extra values masked to 0), so a thread waits twice instead of once per slot; dofs with more
-// than four slots (rare) finish in a loop.
 // Slot sums for dofs with long slot lists: for each round of the thread's dofs, the wave's 64
 // consecutive dofs own one contiguous slot range, which the wave loads coalesced into its LDS
-// row (kWideChunk slots per pass); each lane then adds its own dof's slots from LDS in ascending
+// row (CHUNK slots per pass); each lane then adds its own dof's slots from LDS in ascending
 // order.  Called by every lane of the wave; a dof past the end has the empty range at gptr[n].
 // Latency bounds it (a wave of Q2 vertex dofs owns six times as many slots as the average one), so
 // a pass takes CHUNK slots, CHUNK / 64 loads in flight a lane, and the first 256 of the next round
@@ -488,6 +483,12 @@ template <class T, int CHUNK> __device__ __forceinline__ void gather_slots_wide(
     }
 }
 
+// Slot sums of the ITER dofs a thread of a dof workgroup handles (base + threadIdx.x + m * kBlock),
+// each in ascending slot order; a dof's element outputs sit contiguously in the slot buffer, in
+// ascending cell order.  The slot offsets of all of them are loaded first, then up to four slots
+// each in one wave (indices clamped into the dof's own range, the extra values masked to 0), so a
+// thread waits twice instead of once per slot; dofs with more than four slots (rare) finish in a
+// loop.
 template <class T, int ITER> __device__ __forceinline__ void gather_slots4(const Desc &d, int base, T (&q)[ITER]) {
     const auto Ye = G(reinterpret_cast<const T *>(d.Ye));
     const auto gp = G(d.gptr);
@@ -902,10 +903,10 @@ __device__ __forceinline__ void patch_body(const Desc &d, const ETab &t, int sca
             }
         }
     };
-    // one patch from its loaded tables and node values.  (Loading the next patch's tables ahead, in workgroups of several patches, was
-    // measured: the extra registers cost more resident waves than the hidden latency gained.
-    // Loading only its node ids ahead keeps 8 waves resident and changed nothing: the scattered
-    // node accesses cost memory requests, not latency.)
+    // one patch from its loaded tables and node values.  (Loading the next patch's tables ahead, in
+    // workgroups of several patches, was measured: the extra registers cost more resident waves
+    // than the hidden latency gained.  Loading only its node ids ahead keeps 8 waves resident and
+    // changed nothing: the scattered node accesses cost memory requests, not latency.)
     auto patch = [&](Tables &a, const int p, const int c0, const int nc, const int n0, const int np) {
         const uint4 packed = a.packed;
         const uint4 lent = a.lent;

@@ -681,7 +681,6 @@ Desc q2_desc(fgpu_q2 *s) {
     d.Ye = s->Ye;
     d.q = s->q;
     d.p = s->p;
-    d.z = s->z;
     d.x = s->x;
     d.r = s->r;
     d.zw = s->z;
