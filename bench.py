@@ -724,7 +724,7 @@ def q2_bench(steps: int):
         s1.fill_solution(0.0)
         ctx.sync()
         t0 = time.perf_counter()
-        st1 = s1.solve(fgpu.opts(tol=1e-9, relative=True, precond=fgpu.FGPU_PC_CHEBYSHEV))
+        st1 = s1.solve(fgpu.opts(tol=1e-9, relative=True, precond=fgpu.FGPU_PC_CHEBYSHEV, use_graph=False))
         best = min(best, time.perf_counter() - t0)
     tet_split = q.uses_tet_split()
     ms = q.time_apply(20)

@@ -18,8 +18,11 @@ constexpr int kDofIter = 4;   // dofs per thread in the per-dof kernels
 constexpr int kDofBlock = kBlock * kDofIter;
 // dofs up to which a Q1 system's per-dof kernels run one dof per thread (256 per workgroup): with
 // four, 39k dofs are 38 workgroups on 256 CUs.  One against four, whole calls: 5k dofs 2.40 / 2.74
-// ms, 25k dofs 4.2 / 4.7 ms (mixed), 39k dofs (coupled step) 19.2 / 21.1 ms; 100k dofs gain 3 %, but
-// eight systems of 32k-96k dofs in one batch lose 4 % when all of them run it, 150k dofs lose 1 %
+// ms, 25k dofs 4.2 / 4.7 ms (mixed), 39k dofs (coupled step) 19.2 / 21.1 ms; 100k dofs gain 3 %,
+// 150k dofs lose 1 %, and eight systems of 32k-96k dofs in one batch lose 4 % when all of them run
+// it.  In batches of systems below the line: eight of 32k-43k dofs 8.3 / 8.6 ms (mixed, two-level) and
+// 15.2 / 15.2 (FP64), 32 of 24k-28k dofs 15.0 / 14.6 and 31.8 / 30.8 ms.  A system's own size decides,
+// so that its bits do not depend on its batch.
 constexpr int kSmallDofs = 49152;
 // coarse aggregates of the two-level preconditioner: 2^agg_shift consecutive internal dofs, a
 // multiple of kAggMin (one round of a dof workgroup) and at most its dofs
