@@ -4,8 +4,8 @@ The matrix-free apply processes patches of consecutive cells per workgroup (thei
 staged in LDS); two knobs trade LDS reuse against parallelism and latency hiding:
 cells per patch (the elements-per-block of the element kernel) and patches handled in turn
 by one workgroup.  The best pair depends on the mesh size and on the precision, so it is
-measured on the system's own data: each candidate times whole CG iterations (the patch size
-changes the vector kernel's slots too, and how the iteration's scalars are summed).
+measured on the system's own data: each candidate times the kernels of a CG iteration (the patch
+size changes the vector kernel's slots too, and how the iteration's scalars are summed).
 
 The third knob is the unroll of a batched solve: how many CG iterations are captured in one
 hipGraph between two host convergence checks (more: fewer host round trips; fewer: less

@@ -7,6 +7,7 @@
 #include <cmath>
 #include <cstdio>
 #include <cstring>
+#include <functional>
 #include <mutex>
 #include <new>
 #include <vector>
@@ -2545,10 +2546,12 @@ extern "C" int fgpu_sys_solve(fgpu_sys *s, const fgpu_solve_opts *o, fgpu_solve_
 // kernel of a CG iteration, measured with HIP events on the context stream
 // ------------------------------------------------------------------------------------------
 // average duration of `reps` back-to-back launches of the element apply (which 0), the vector work
-// (which 1) or the coarse product of the two-level FP32 CG (which 2), or of `reps` whole iterations
-// (which 3), HIP events on the context's stream.  The kernels and descriptors are those of the CG, in
-// an iteration that neither starts nor stops; what a later iteration reads (state, partials, vectors,
-// coarse corrections) is kept in copies, so that a running solve goes on undisturbed.
+// (which 1) or the coarse product of the two-level FP32 CG (which 2), or the sum of these and the
+// scalar kernels over one iteration (which 3; timed one by one, so that a host slower than the
+// kernels does not set it), HIP events on the context's stream.  The kernels and descriptors are those
+// of the CG, in an iteration that neither starts nor stops; what a later iteration reads (state,
+// partials, vectors, coarse corrections) is kept in copies, so that a running solve goes on
+// undisturbed.
 static double time_launches(fgpu_ctx *c, const std::vector<fgpu_sys *> &sys, const fgpu_solve_opts *o, bool coef, int which,
                             int reps) {
     const bool mixed = o->precision == FGPU_MIXED;
@@ -2583,35 +2586,40 @@ static double time_launches(fgpu_ctx *c, const std::vector<fgpu_sys *> &sys, con
     }
     BatchTabs t = upload_batch(c, sets, sys);
     if (which == 2 && (!mixed || t.nct == 0)) throw std::invalid_argument("no coarse level in the batch");
-    const Desc *D = t.sets[mixed ? 2 : 0];
-    auto one = [&] {
-        if (which == 2) {
-            launch_coarse(st, D, nullptr, t.ctab, t.nct, 0, t.host(D));
-        } else if (which == 3) {
-            if (mixed) cg_iter<float>(st, D, nullptr, t, (int)sys.size(), kind, 1, false);
-            else cg_iter<double>(st, D, nullptr, t, (int)sys.size(), kind, 0, false);
-        } else if (which == 0) {
-            if (mixed) cg_apply<float>(st, D, t, coef);
-            else cg_apply<double>(st, D, t, coef);
-        } else {
-            if (mixed) cg_vectors<float>(st, D, t);
-            else cg_vectors<double>(st, D, t);
-        }
+    const Desc *D = t.sets[mixed ? 2 : 0], *one = t.host(D);
+    const int n = (int)sys.size();
+    using Launch = std::function<void()>;
+    const Launch apply = [&] { mixed ? cg_apply<float>(st, D, t, coef) : cg_apply<double>(st, D, t, coef); };
+    const Launch vectors = [&] { mixed ? cg_vectors<float>(st, D, t) : cg_vectors<double>(st, D, t); };
+    const Launch coarse = [&] {
+        if (mixed) launch_coarse(st, D, nullptr, t.ctab, t.nct, 0, one);
+        else if (kind.coarse64) launch_coarse64(st, D, t.ctab, t.nct, one);
     };
-    one();
+    std::vector<Launch> launches;
+    if (which == 0) launches = {apply};
+    else if (which == 2) launches = {coarse};
+    else if (which != 3) launches = {vectors};
+    else if (t.fold) launches = {apply, vectors, coarse};
+    else launches = {apply, [&] { launch_scal_alpha(st, D, n, one); }, vectors, coarse,
+                     [&] { launch_scal_beta(st, D, n, mixed ? 1 : 0, false, one); }};
     hipEvent_t e0, e1;
     HIPCHECK(hipEventCreate(&e0));
     HIPCHECK(hipEventCreate(&e1));
-    HIPCHECK(hipEventRecord(e0, st));
-    for (int i = 0; i < reps; ++i) one();
-    HIPCHECK(hipEventRecord(e1, st));
-    HIPCHECK(hipEventSynchronize(e1));
-    HIPCHECK(hipGetLastError());
-    float ms = 0;
-    HIPCHECK(hipEventElapsedTime(&ms, e0, e1));
+    double total = 0.0;
+    for (const Launch &launch : launches) {
+        launch();
+        HIPCHECK(hipEventRecord(e0, st));
+        for (int i = 0; i < reps; ++i) launch();
+        HIPCHECK(hipEventRecord(e1, st));
+        HIPCHECK(hipEventSynchronize(e1));
+        HIPCHECK(hipGetLastError());
+        float ms = 0;
+        HIPCHECK(hipEventElapsedTime(&ms, e0, e1));
+        total += ms;
+    }
     (void)hipEventDestroy(e0);
     (void)hipEventDestroy(e1);
-    return ms / reps;
+    return total / reps;
 }
 
 extern "C" int fgpu_sys_time_kernel(fgpu_sys *s, int which, int precision, int reps, double *avg_ms) {

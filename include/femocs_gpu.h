@@ -246,8 +246,9 @@ int fgpu_batch_step_async(fgpu_batch *batch, int iterations);
 int fgpu_batch_wait(fgpu_batch *batch, int *n_running);
 /* average duration (ms) of one launch of a CG iteration's element apply (which 0), vector work
  * (which 1) or coarse product of the two-level preconditioner (which 2, mixed batches with a
- * coarse level), or of one whole iteration (which 3), over all members, in the batch's precision;
- * for measurement, no counterpart in the reference.  Running solves go on undisturbed. */
+ * coarse level), or the sum over the launches of one iteration (which 3), over all members, in the
+ * batch's precision; for measurement, no counterpart in the reference.  Running solves go on
+ * undisturbed. */
 int fgpu_batch_time_kernel(fgpu_batch *batch, int which, int reps, double *avg_ms);
 /* ---- transfer to atoms (Interpolator, InterpolatorCells, SolutionReader) ---------------
  * An interpolator holds the tet mesh, its Tethex hexes (4 per tet, hex 4t+k around vertex k,
